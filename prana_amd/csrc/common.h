@@ -131,15 +131,11 @@ static __constant__ const uint64_t kExp2Tab[32] = {
     0x3fef5818dcfba487ull, 0x3fef7c97337b9b5full, 0x3fefa4afa2a490daull, 0x3fefd0765b6e4540ull,
 };
 
-__device__ __forceinline__ float dev_expf(float x) {
-  uint32_t ux = __float_as_uint(x);
-  uint32_t abstop = (ux >> 20) & 0x7ffu;
-  if (abstop >= 0x42bu) {                       // |x| >= 88 or x is NaN/inf
-    if (ux == 0xff800000u) return 0.0f;         // exp(-inf)
-    if (abstop >= 0x7f8u) return x + x;         // +inf or NaN
-    if (x > 0x1.62e42ep6f) return __uint_as_float(0x7f800000u);  // overflow
-    if (x < -0x1.9fe368p6f) return 0.0f;                          // underflow
-  }
+// tab: kExp2Tab, or a workgroup's copy of it in LDS (its 32 entries fall on
+// distinct banks, so a wave's lookups cost one LDS read instead of a gather
+// through the vector cache). The special cases are selects, not branches:
+// callers evaluate many values per lane.
+__device__ __forceinline__ float dev_expf_tab(float x, const uint64_t* tab) {
   const double kInvLn2N = 0x1.71547652b82fep+0 * 32.0;
   const double kShift = 0x1.8p+52;
   const double c0 = 0x1.c6af84b912394p-5 / 32.0 / 32.0 / 32.0;
@@ -150,15 +146,20 @@ __device__ __forceinline__ float dev_expf(float x) {
   uint64_t ki = static_cast<uint64_t>(__double_as_longlong(kd));
   kd -= kShift;
   double r = __fma_rn(kInvLn2N, xd, -kd);
-  uint64_t t = kExp2Tab[ki % 32] + (ki << 47);
+  uint64_t t = tab[ki % 32] + (ki << 47);
   double s = __longlong_as_double(static_cast<long long>(t));
   double z = __fma_rn(c0, r, c1);
   double r2 = r * r;
   double y = __fma_rn(c2, r, 1.0);
   y = __fma_rn(z, r2, y);
   y = y * s;
-  return static_cast<float>(y);
+  float e = static_cast<float>(y);
+  e = x > 0x1.62e42ep6f ? __uint_as_float(0x7f800000u) : e;  // overflow, +inf
+  e = x < -0x1.9fe368p6f ? 0.0f : e;                          // underflow, -inf
+  return x != x ? x + x : e;                                  // NaN
 }
+
+__device__ __forceinline__ float dev_expf(float x) { return dev_expf_tab(x, kExp2Tab); }
 
 // ---------------------------------------------------------------- tanhf
 // gelu_tanh (norms.rs:35-41) reaches tanhf through Rust's f32::tanh ->

@@ -247,6 +247,16 @@ int launch_attention_prefill(const float* q, const float* k, const float* v, siz
                              size_t n_kv_heads, size_t hd, float* out, float* scratch, hipStream_t s,
                              const ActQuant* aq = nullptr, bool* quantized = nullptr);
 
+// ---- prefill_attention.hip
+// The tiled prefill attention: 16-byte aligned q, k and v, head widths that
+// are multiples of 4 up to 256, and enough query rows (prefill_tile_takes).
+// scratch >= prefill_tile_scratch_floats(seq, n_heads) floats.
+size_t prefill_tile_scratch_floats(size_t seq, size_t n_heads);
+bool prefill_tile_takes(const float* q, const float* k, const float* v, size_t seq, size_t n_heads, size_t hd);
+int launch_prefill_tile(const float* q, const float* k, const float* v, size_t seq, size_t n_heads,
+                        size_t n_kv_heads, size_t hd, float* out, float* scratch, const ActQuant* aq,
+                        bool* quantized, hipStream_t s);
+
 // ---- flash_decode.hip
 // Split-K flash decoding (attention_decode, attention.rs:129-195, for up to 16
 // independent sequences; f32 within 1e-4 relative, not bit-exact). The plan

@@ -1,0 +1,50 @@
+"""Tiled prefill attention (prefill_attention.hip) against the oracle's
+`attention` (attention.rs:236-284), bit for bit: block and tile edges (16 / 32 / 64
+query rows, 128 / 256 keys), head widths that fill a lane tile or leave part
+of it empty, several blocks per workgroup, and non-finite K and V rows."""
+import numpy as np
+import pytest
+
+import prana_amd as P
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def same_bits(a, b):
+    return np.array_equal(np.asarray(a, np.float32).view(np.uint32), np.asarray(b, np.float32).view(np.uint32))
+
+
+def qkv(seq, nh, nkv, hd):
+    r = np.random.default_rng(seq * 1000 + hd)
+    return [r.standard_normal(seq * n * hd).astype(np.float32) for n in (nh, nkv, nkv)]
+
+
+# (seq, query heads, KV heads, head width), by query rows per block: 16 (the
+# first group; lane tiles filled or partly empty, edges of 16 rows, 64-key
+# groups and 256-key tiles), 32 (from 640 such blocks), 64 (from 1024)
+@pytest.mark.parametrize("seq,nh,nkv,hd", [
+    (16, 44, 4, 64), (17, 48, 48, 4), (63, 16, 2, 128), (65, 12, 6, 48), (129, 8, 1, 20), (257, 5, 5, 256),
+    (200, 5, 5, 80), (255, 3, 1, 96), (256, 8, 8, 100), (300, 4, 1, 132), (1000, 14, 2, 64),
+    (350, 64, 8, 64), (321, 64, 16, 128), (319, 64, 64, 8), (330, 60, 4, 160),
+    (513, 128, 8, 64), (520, 128, 16, 72), (1025, 64, 8, 12)])
+def test_prefill_tile(seq, nh, nkv, hd):
+    q, k, v = qkv(seq, nh, nkv, hd)
+    assert same_bits(P.attention_prefill(q, k, v, seq, nh, nkv, hd), O.attention(q, k, v, seq, nh, nkv, hd))
+
+
+def test_prefill_tile_nonfinite():
+    # a key's infinite or NaN row must not reach the rows before it, whose
+    # products never include it
+    seq, nh, nkv, hd = 150, 6, 1, 64
+    q, k, v = qkv(seq, nh, nkv, hd)
+    v = v.reshape(seq, hd)
+    v[40, 3], v[70, 5], v[100, 7] = np.inf, np.nan, -np.inf
+    k = k.reshape(seq, hd)
+    k[120] = np.nan
+    k[130, 0] = np.inf
+    got = P.attention_prefill(q, k, v, seq, nh, nkv, hd)
+    want = O.attention(q, k.ravel(), v.ravel(), seq, nh, nkv, hd)
+    gn, wn = np.isnan(got), np.isnan(want)
+    assert np.array_equal(gn, wn)  # NaN payloads are not part of the contract
+    assert np.array_equal(got[~gn].view(np.uint32), want[~wn].view(np.uint32))
