@@ -320,33 +320,6 @@ int launch_act_mul(float* g, const float* u, size_t n, int gelu, int8_t* q, floa
   return kOk;
 }
 
-// ---------------------------------------------------------------- softmax
-// norms.rs:44-56, one workgroup per row; the sum is the sequential fold,
-// evaluated exactly by the workgroup.
-__global__ __launch_bounds__(256) void softmax_kernel(const float* __restrict__ in, int n, float* __restrict__ out) {
-  __shared__ float s_red[4];
-  const float* row = in + (size_t)blockIdx.x * n;
-  float* dst = out + (size_t)blockIdx.x * n;
-  float mx = -INFINITY;
-  for (int i = threadIdx.x; i < n; i += 256) mx = fmaxf(mx, row[i]);
-  mx = wave_max_f32(mx);
-  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = mx;
-  __syncthreads();
-  mx = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-  for (int i = threadIdx.x; i < n; i += 256) dst[i] = dev_expf(row[i] - mx);
-  __syncthreads();
-  const float sum = exact::block_seq_sum_nonneg<256, false>(dst, n);  // norms.rs:53 order
-  const float inv = sum > 0.0f ? 1.0f / sum : 0.0f;
-  for (int i = threadIdx.x; i < n; i += 256) dst[i] = dst[i] * inv;
-}
-
-int launch_softmax(const float* in, size_t rows, size_t n, float* out, hipStream_t s) {
-  if (rows == 0 || n == 0) return kOk;
-  hipLaunchKernelGGL(softmax_kernel, dim3(rows), dim3(256), 0, s, in, (int)n, out);
-  PRANA_LAUNCH_CHECK();
-  return kOk;
-}
-
 // ---------------------------------------------------------------- add
 __global__ void add_kernel(float* __restrict__ x, const float* __restrict__ y, size_t n, size_t period) {
   size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x;

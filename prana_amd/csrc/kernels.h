@@ -44,7 +44,6 @@ int launch_quantize_acts(const float* x, size_t n_rows, size_t k, int8_t* q, flo
 int launch_rmsnorm(const float* x, const float* w, size_t rows, size_t dim, float eps, float* out, int8_t* q,
                    float* sa, int* sums, hipStream_t s);
 int launch_act_mul(float* g, const float* u, size_t n, int gelu, int8_t* q, float* sa, int* sums, hipStream_t s);
-int launch_softmax(const float* in, size_t rows, size_t n, float* out, hipStream_t s);
 int launch_add(float* x, const float* y, size_t n, size_t period, hipStream_t s);
 int launch_rope(float* x, size_t n_rows, size_t row_len, size_t row_stride, size_t hd, const float2* table,
                 size_t pos0, int neox, hipStream_t s);
@@ -74,6 +73,9 @@ int launch_decode_seed(int* state, int pos, uint32_t token, uint32_t* ids, uint3
 // target argmaxes tnext[0..budget]; res = {emitted, accepted, done, tokens...}.
 int launch_spec_accept(const uint32_t* drafts, const uint32_t* tnext, int budget, const uint32_t* stops, int n_stops,
                        size_t generated, size_t steps, size_t pos, size_t max_pos, int* res, hipStream_t s);
+
+// ---- softmax.hip
+int launch_softmax(const float* in, size_t rows, size_t n, float* out, hipStream_t s);
 
 // ---- sampler.hip
 // Sampler::sample's bucket walk (sampler.rs:29-36) over device probabilities:

@@ -1,5 +1,5 @@
 // Temperature sampling (Sampler::sample, sampler.rs:22-39) on the device:
-// logits / temp, the exact softmax (softmax_kernel), then the bucket walk
+// logits / temp, the exact softmax (softmax.hip), then the bucket walk
 //   r = u01; for i: r -= p[i]; if r <= 0 return i;   (last index otherwise)
 // in the reference's left-to-right f32 order.
 //
