@@ -1800,31 +1800,6 @@ __global__ __launch_bounds__(256) void isums_kernel(DevMat m, const int8_t* __re
     F::isums(m, r, b, a, out + ((size_t)tok * m.rows + r) * T + b * F::kTpu);
 }
 
-// Dense f32 rows: dot_f32_scalar (matmul.rs:377-391) — four strided partial
-// sums, combined ((a0+a1)+a2)+a3, then the tail. One lane per partial sum.
-__global__ __launch_bounds__(256) void gemv_f32_kernel(DevMat m, const float* __restrict__ x, GemvOut o) {
-  __shared__ float part[256];
-  const int K = static_cast<int>(m.cols);
-  const int tok = blockIdx.y;
-  const int rr = threadIdx.x >> 2, l = threadIdx.x & 3;
-  const size_t r = (size_t)blockIdx.x * 64 + rr;
-  const float* xr = x + (size_t)tok * K;
-  float acc = 0.0f;
-  if (r < m.rows) {
-    const float* w = reinterpret_cast<const float*>(m.qs) + r * K;
-    const int chunks = K / 4;
-    for (int i = 0; i < chunks; i++) acc += xr[i * 4 + l] * w[i * 4 + l];
-  }
-  part[threadIdx.x] = acc;
-  __syncthreads();
-  if (l == 0 && r < m.rows) {
-    const float* w = reinterpret_cast<const float*>(m.qs) + r * K;
-    float sum = part[threadIdx.x] + part[threadIdx.x + 1] + part[threadIdx.x + 2] + part[threadIdx.x + 3];
-    for (int i = (K / 4) * 4; i < K; i++) sum += xr[i] * w[i];
-    store_out(o, tok, r, sum);
-  }
-}
-
 // ===================================================================
 // Batched matmul on the int8 matrix cores (prefill / verify, N > 16 tokens).
 // Q4_0 needs no activation sums here: its nibbles enter the matrix cores as
@@ -3346,13 +3321,7 @@ int launch_gemv(const DevMat& m, const float* x, const int8_t* q, const float* s
     return dispatch_kind(m.kind, [&](auto k) { return launch_decode_t<decltype(k)::value>(job, q, sa, sums, n_tok, s); });
   }
   switch (m.kind) {
-    case kKindF32: {
-      PRANA_CHECK(x != nullptr, "gemv f32: dense activations required");
-      dim3 grid((m.rows + 63) / 64, n_tok);
-      hipLaunchKernelGGL(gemv_f32_kernel, grid, dim3(256), 0, s, m, x, o);
-      PRANA_LAUNCH_CHECK();
-      return kOk;
-    }
+    case kKindF32: return launch_gemv_f32(m, x, n_tok, o, s);
     case kKindQ8F: return launch_gemm_mfma<kKindQ8F>(&m, &o, 1, q, sa, n_tok, s);
     case kKindQ8_0: return launch_gemm_mfma<kKindQ8_0>(&m, &o, 1, q, sa, n_tok, s);
     case kKindQ4_0: return launch_gemm_mfma<kKindQ4_0>(&m, &o, 1, q, sa, n_tok, s);

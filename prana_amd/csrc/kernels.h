@@ -214,6 +214,10 @@ int launch_gemv_act(const DevMat& gate, const DevMat& up, int act, const int8_t*
 int launch_block_isums(const DevMat& m, const int8_t* q, const int* sums, size_t n_tok, int* isums, hipStream_t s);
 size_t terms_per_row(const DevMat& m);
 
+// ---- dense.hip
+// Linear::F32 (matmul_f32, matmul.rs:150-157) for n_tok rows of x.
+int launch_gemv_f32(const DevMat& m, const float* x, size_t n_tok, const GemvOut& o, hipStream_t s);
+
 // ---- attention.hip
 // attention_decode / attention_verify (attention.rs:129-160, 296-333) over the
 // f16 cache: n_q query rows at positions pos0 + i (pos0 read from pos_dev when
