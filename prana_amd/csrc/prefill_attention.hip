@@ -27,7 +27,7 @@
 // its L2.
 //
 // Measured (one MI355X, one call): 14 heads x 64 dims at 2048 positions 275
-// us and at 3001 575 us, 32 heads x 128 at 2048 963 us; the kernels before
+// us and at 3001 505 us, 32 heads x 128 at 2048 963 us; the kernels before
 // took 550 (eight query rows per workgroup, one key row gathered per lane),
 // 5590 and 1760. At 32 x 128 x 2048 the counters show the vector ALU issuing
 // in every cycle, 17 % of its instructions not products or sums of the two
@@ -76,8 +76,8 @@ __host__ __device__ constexpr size_t pt_stride(size_t seq) { return (seq + kPtTK
 
 // scratch: gridDim.x slots of BQ rows of sstride floats. nx: 8 when heads are
 // dealt to the XCDs, else 1 (gridDim.x is a multiple of nx).
-template <int BQ, int HDP>
-__global__ __launch_bounds__(kPtNT, BQ == 16 ? 3 : 2) void attn_prefill_tile(const float* __restrict__ q, const float* __restrict__ k,
+template <int BQ, int HDP, int WPC>
+__global__ __launch_bounds__(kPtNT, WPC) void attn_prefill_tile(const float* __restrict__ q, const float* __restrict__ k,
                                                            const float* __restrict__ v, int seq, int n_heads,
                                                            int group, int hd, float* __restrict__ out,
                                                            float* __restrict__ scratch, int sstride,
@@ -395,7 +395,7 @@ __global__ __launch_bounds__(kPtNT, BQ == 16 ? 3 : 2) void attn_prefill_tile(con
 // product, but the placement of workgroups is not ours, so a launch of one
 // round leaves compute units with unequal blocks. Blocks of 64 rows are
 // taken once every slot gets two (2048 positions of 32 heads: 963 us), of 32
-// rows from 2.5 per compute unit (1024 positions: 289 us against 437 with 64
+// rows from 2.5 per compute unit (1024 positions: 254 us against 437 with 64
 // rows; 800: 204 against 252 with 16), else 16 (511: 96 us against 133 with
 // 32).
 int pt_block(size_t seq, size_t n_heads) {
@@ -403,19 +403,28 @@ int pt_block(size_t seq, size_t n_heads) {
   return jobs(64) >= 4 * kPtCus ? 64 : jobs(32) >= kPtCus * 5 / 2 ? 32 : 16;
 }
 
-// Workgroups, each with a scratch slot: as many as are resident (three per
-// compute unit with 16-row blocks, two beyond: 511 positions of 32 heads 96
-// against 120 us with two).
-size_t pt_slots(int bq, size_t seq, size_t n_heads) {
-  return std::min((seq + bq - 1) / bq * n_heads, size_t{kPtCus} * (bq == 16 ? 3 : 2));
+// Workgroups per compute unit (compiled for that many, and as many slots).
+// Three from about four blocks per compute unit on, where LDS allows (14 heads
+// x 64 at 3001 positions 505 us against 575 with two; 32 x 128 at 1024 254
+// against 289); with fewer blocks the registers that two leave free are worth
+// more (14 x 64 at 2048 275 against 299). 16-row blocks always take three (32 x
+// 128 at 511 96 against 120; 8 x 256 at 1500 367 against 395, though only two
+// fit).
+int pt_wpc(int bq, size_t seq, size_t n_heads, size_t hd) {
+  if (bq == 16) return 3;
+  // (64-row blocks are taken from 1024 on)
+  return hd <= (bq == 64 ? 64u : 128u) && (seq + bq - 1) / bq * n_heads >= 1000 ? 3 : 2;
+}
+size_t pt_slots(int bq, int wpc, size_t seq, size_t n_heads) {
+  return std::min((seq + bq - 1) / bq * n_heads, size_t{kPtCus} * wpc);
 }
 
-template <int BQ, int HDP>
+template <int BQ, int HDP, int WPC>
 int launch_tile(const float* q, const float* k, const float* v, size_t seq, size_t n_heads, size_t n_kv_heads,
                 size_t hd, float* out, float* scratch, const ActQuant* aq, hipStream_t s) {
   const int nx = n_heads % 8 == 0 ? 8 : 1;
-  const size_t grid = pt_slots(BQ, seq, n_heads);  // a multiple of nx
-  hipLaunchKernelGGL((attn_prefill_tile<BQ, HDP>), dim3(grid), dim3(kPtNT), 0, s, q, k, v, (int)seq, (int)n_heads,
+  const size_t grid = pt_slots(BQ, WPC, seq, n_heads);  // a multiple of nx
+  hipLaunchKernelGGL((attn_prefill_tile<BQ, HDP, WPC>), dim3(grid), dim3(kPtNT), 0, s, q, k, v, (int)seq, (int)n_heads,
                      (int)(n_heads / n_kv_heads), (int)hd, out, scratch, (int)pt_stride(seq), aq ? aq->q : nullptr,
                      aq ? aq->sa : nullptr, aq ? aq->sums : nullptr, nx);
   PRANA_LAUNCH_CHECK();
@@ -426,7 +435,7 @@ int launch_tile(const float* q, const float* k, const float* v, size_t seq, size
 
 size_t prefill_tile_scratch_floats(size_t seq, size_t n_heads) {
   const int bq = pt_block(seq, n_heads);  // (wide heads take 32 rows where others take 64: less)
-  return pt_slots(bq, seq, n_heads) * bq * pt_stride(seq);
+  return pt_slots(bq, 3, seq, n_heads) * bq * pt_stride(seq);
 }
 
 // Below these (query row, head) counts the one-launch kernel's workgroup per
@@ -446,12 +455,17 @@ int launch_prefill_tile(const float* q, const float* k, const float* v, size_t s
   const ActQuant* fuse = aq && aq->q && hd % 32 == 0 ? aq : nullptr;
   if (quantized) *quantized = fuse != nullptr;
   const int bq = pt_block(seq, n_heads);
+  const bool three = pt_wpc(bq, seq, n_heads, hd) == 3;
   auto go = [&](auto hdp) {
     constexpr int HDP = decltype(hdp)::value;
-    if constexpr (HDP <= 128)
-      if (bq == 64) return launch_tile<64, HDP>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
-    if (bq >= 32) return launch_tile<32, HDP>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
-    return launch_tile<16, HDP>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
+    if constexpr (HDP <= 128) {
+      if (bq == 64)
+        return launch_tile<64, HDP, HDP == 64 ? 3 : 2>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
+      if (bq == 32 && three)
+        return launch_tile<32, HDP, 3>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
+    }
+    if (bq >= 32) return launch_tile<32, HDP, 2>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
+    return launch_tile<16, HDP, 3>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
   };
   if (hd > 128) return go(std::integral_constant<int, 256>());
   if (hd > 64) return go(std::integral_constant<int, 128>());

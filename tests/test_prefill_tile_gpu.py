@@ -22,11 +22,13 @@ def qkv(seq, nh, nkv, hd):
 
 # (seq, query heads, KV heads, head width), by query rows per block: 16 (the
 # first group; lane tiles filled or partly empty, edges of 16 rows, 64-key
-# groups and 256-key tiles), 32 (from 640 such blocks), 64 (from 1024)
+# groups and 256-key tiles), 32 (from 640 such blocks, compiled for three
+# workgroups per compute unit from 1000), 64 (from 1024)
 @pytest.mark.parametrize("seq,nh,nkv,hd", [
     (16, 44, 4, 64), (17, 48, 48, 4), (63, 16, 2, 128), (65, 12, 6, 48), (129, 8, 1, 20), (257, 5, 5, 256),
     (200, 5, 5, 80), (255, 3, 1, 96), (256, 8, 8, 100), (300, 4, 1, 132), (1000, 14, 2, 64),
     (350, 64, 8, 64), (321, 64, 16, 128), (319, 64, 64, 8), (330, 60, 4, 160),
+    (350, 96, 8, 48), (340, 96, 12, 72),
     (513, 128, 8, 64), (520, 128, 16, 72), (1025, 64, 8, 12)])
 def test_prefill_tile(seq, nh, nkv, hd):
     q, k, v = qkv(seq, nh, nkv, hd)
