@@ -1284,15 +1284,25 @@ int attention_dim_slices(size_t n_q, size_t n_heads, size_t hd, size_t elem, boo
 
 bool attention_split_window(size_t rows, size_t hd) { return rows >= kSplitMinRows && (hd == 64 || hd == 128); }
 
-size_t attention_scratch_floats(size_t n_q, size_t n_heads, size_t ctx_cap, bool cache) {
-  // split path (cache windows): scores / probabilities of every (query row, head)
-  size_t need = cache ? n_q * n_heads * split_stride(ctx_cap) : prefill_tile_scratch_floats(ctx_cap, n_heads);
-  if (ctx_cap > static_cast<size_t>(kScoreLds)) {
-    size_t ds = 1;  // upper bound of attention_dim_slices
-    while (n_q * n_heads * ds < 128 && ds < 4) ds *= 2;
-    need = std::max(need, n_q * n_heads * ds * ctx_cap);
-  }
-  return need;
+// Score rows of the one-launch kernel past the LDS (attention.hip's attn_kernel).
+static size_t spill_floats(size_t n_q, size_t n_heads, size_t ctx_cap) {
+  if (ctx_cap <= static_cast<size_t>(kScoreLds)) return 0;
+  size_t ds = 1;  // upper bound of attention_dim_slices
+  while (n_q * n_heads * ds < 128 && ds < 4) ds *= 2;
+  return n_q * n_heads * ds * ctx_cap;
+}
+
+size_t attention_scratch_floats(size_t n_q, size_t n_heads, size_t ctx_cap) {
+  // split path: scores / probabilities of every (query row, head)
+  return std::max(n_q * n_heads * split_stride(ctx_cap), spill_floats(n_q, n_heads, ctx_cap));
+}
+
+// Sized by the kernel that takes the shape: a long prompt on the tiled kernel
+// needs its slots only (32 heads x 16384 positions 3.2 GB), not the one-launch
+// kernel's score rows (34 GB).
+size_t attention_prefill_scratch_floats(size_t seq, size_t n_heads, size_t hd, bool aligned) {
+  if (aligned && prefill_tile_takes(seq, n_heads, hd)) return prefill_tile_scratch_floats(seq, n_heads, hd);
+  return spill_floats(seq, n_heads, seq);
 }
 
 int launch_attention_cache(const float* q, const uint16_t* kc, const uint16_t* vc, size_t pos0, size_t n_q,
@@ -1313,7 +1323,7 @@ int launch_attention_prefill(const float* q, const float* k, const float* v, siz
   if (seq == 0) return kOk;
   PRANA_CHECK(n_kv_heads > 0 && n_heads % n_kv_heads == 0, "attention: n_heads must be a multiple of n_kv_heads");
   PRANA_CHECK(hd > 0 && hd <= 256, "attention: head_dim must be in 1..=256");
-  if (scratch && prefill_tile_takes(q, k, v, seq, n_heads, hd))
+  if (scratch && prefill_tile_takes(seq, n_heads, hd) && prefill_tile_aligned(q, k, v))
     return launch_prefill_tile(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, aq, quantized, s);
   return launch_attn<false>(q, k, v, 0, nullptr, seq, n_heads, n_kv_heads, hd, out, scratch, seq, aq, quantized, 0, s);
 }

@@ -160,7 +160,8 @@ int Graph::execute(hipStream_t s, int* kind, size_t* node) {
     if (n.has_value) continue;
     if (n.op == GraphNode::kMatmulQ8) q_elems = std::max(q_elems, n_tokens * n.w->d.cols);
     if (n.op == GraphNode::kAttention)
-      att_floats = std::max(att_floats, attention_scratch_floats(n_tokens, n.n_heads, n_tokens, false));
+      att_floats = std::max(att_floats,  // (values are allocations: aligned)
+                            attention_prefill_scratch_floats(n_tokens, n.n_heads, n.head_dim, true));
   }
   int rc;
   if (q_elems && ((rc = qa.ensure(q_elems)) || (rc = sa.ensure(q_elems / 32 * 4)) || (rc = sums.ensure(q_elems / 32 * 4))))

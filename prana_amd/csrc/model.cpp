@@ -251,7 +251,8 @@ int Model::ensure_ws(size_t n_tok, size_t ctx_cap, bool prefill_attn) {
     PRANA_HIP(hipMemset(ws.xch.p, 0, ws.xch.bytes));
     ws.gen++;
   }
-  size_t need = (prefill_attn ? attention_scratch_floats(n_tok, c.n_heads, n_tok, false)
+  // (the workspace's q, k and v are allocations: aligned)
+  size_t need = (prefill_attn ? attention_prefill_scratch_floats(n_tok, c.n_heads, c.head_dim, true)
                               : attention_scratch_floats(n_tok, c.n_heads, ctx_cap)) * 4;
   const void* before = ws.scratch.p;
   if ((rc = ws.scratch.ensure(std::max<size_t>(need, 4)))) return rc;

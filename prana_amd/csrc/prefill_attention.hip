@@ -419,6 +419,18 @@ size_t pt_slots(int bq, int wpc, size_t seq, size_t n_heads) {
   return std::min((seq + bq - 1) / bq * n_heads, size_t{kPtCus} * wpc);
 }
 
+// The launch a shape takes: query rows per block, padded head width,
+// workgroups per compute unit.
+struct PtPlan {
+  int bq, hdp, wpc;
+};
+PtPlan pt_plan(size_t seq, size_t n_heads, size_t hd) {
+  const int bq = pt_block(seq, n_heads), hdp = hd > 128 ? 256 : hd > 64 ? 128 : 64;
+  if (bq == 16) return PtPlan{16, hdp, 3};
+  if (hdp == 256) return PtPlan{32, hdp, 2};  // (wide heads have no 64-row instance)
+  return PtPlan{bq, hdp, pt_wpc(bq, seq, n_heads, hd)};
+}
+
 template <int BQ, int HDP, int WPC>
 int launch_tile(const float* q, const float* k, const float* v, size_t seq, size_t n_heads, size_t n_kv_heads,
                 size_t hd, float* out, float* scratch, const ActQuant* aq, hipStream_t s) {
@@ -433,42 +445,45 @@ int launch_tile(const float* q, const float* k, const float* v, size_t seq, size
 
 }  // namespace
 
-size_t prefill_tile_scratch_floats(size_t seq, size_t n_heads) {
-  const int bq = pt_block(seq, n_heads);  // (wide heads take 32 rows where others take 64: less)
-  return pt_slots(bq, 3, seq, n_heads) * bq * pt_stride(seq);
+size_t prefill_tile_scratch_floats(size_t seq, size_t n_heads, size_t hd) {
+  const PtPlan p = pt_plan(seq, n_heads, hd);
+  return pt_slots(p.bq, p.wpc, seq, n_heads) * p.bq * pt_stride(seq);
 }
 
 // Below these (query row, head) counts the one-launch kernel's workgroup per
 // row and head is faster: 14 heads x 32 positions 21 against 26 us, 6 x 100
 // 26 against 28, 16 x 50 32 against 29, 32 x 32 34 against 31; 256-wide
 // heads, 8 x 120 61 against 67, 8 x 300 211 against 111.
-bool prefill_tile_takes(const float* q, const float* k, const float* v, size_t seq, size_t n_heads, size_t hd) {
+bool prefill_tile_takes(size_t seq, size_t n_heads, size_t hd) {
+  return hd % 4 == 0 && hd <= 256 && seq >= 16 && seq * n_heads >= (hd <= 128 ? 700u : 1100u) &&
+         seq <= static_cast<size_t>(INT32_MAX) / 2;
+}
+bool prefill_tile_aligned(const float* q, const float* k, const float* v) {
   return reinterpret_cast<uintptr_t>(q) % 16 == 0 && reinterpret_cast<uintptr_t>(k) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(v) % 16 == 0 && hd % 4 == 0 && hd <= 256 && seq >= 16 &&
-         seq * n_heads >= (hd <= 128 ? 700u : 1100u) && seq <= static_cast<size_t>(INT32_MAX) / 2;
+         reinterpret_cast<uintptr_t>(v) % 16 == 0;
 }
 
 int launch_prefill_tile(const float* q, const float* k, const float* v, size_t seq, size_t n_heads,
                         size_t n_kv_heads, size_t hd, float* out, float* scratch, const ActQuant* aq,
                         bool* quantized, hipStream_t s) {
-  PRANA_CHECK(prefill_tile_takes(q, k, v, seq, n_heads, hd) && scratch, "prefill attention: shape out of range");
+  PRANA_CHECK(prefill_tile_takes(seq, n_heads, hd) && prefill_tile_aligned(q, k, v) && scratch,
+              "prefill attention: shape out of range");
   const ActQuant* fuse = aq && aq->q && hd % 32 == 0 ? aq : nullptr;
   if (quantized) *quantized = fuse != nullptr;
-  const int bq = pt_block(seq, n_heads);
-  const bool three = pt_wpc(bq, seq, n_heads, hd) == 3;
+  const PtPlan p = pt_plan(seq, n_heads, hd);
   auto go = [&](auto hdp) {
     constexpr int HDP = decltype(hdp)::value;
     if constexpr (HDP <= 128) {
-      if (bq == 64)
+      if (p.bq == 64)
         return launch_tile<64, HDP, HDP == 64 ? 3 : 2>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
-      if (bq == 32 && three)
+      if (p.bq == 32 && p.wpc == 3)
         return launch_tile<32, HDP, 3>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
     }
-    if (bq >= 32) return launch_tile<32, HDP, 2>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
+    if (p.bq == 32) return launch_tile<32, HDP, 2>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
     return launch_tile<16, HDP, 3>(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, fuse, s);
   };
-  if (hd > 128) return go(std::integral_constant<int, 256>());
-  if (hd > 64) return go(std::integral_constant<int, 128>());
+  if (p.hdp == 256) return go(std::integral_constant<int, 256>());
+  if (p.hdp == 128) return go(std::integral_constant<int, 128>());
   return go(std::integral_constant<int, 64>());
 }
 
