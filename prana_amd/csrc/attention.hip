@@ -1323,7 +1323,7 @@ int launch_attention_prefill(const float* q, const float* k, const float* v, siz
   if (seq == 0) return kOk;
   PRANA_CHECK(n_kv_heads > 0 && n_heads % n_kv_heads == 0, "attention: n_heads must be a multiple of n_kv_heads");
   PRANA_CHECK(hd > 0 && hd <= 256, "attention: head_dim must be in 1..=256");
-  if (scratch && prefill_tile_takes(seq, n_heads, hd) && prefill_tile_aligned(q, k, v))
+  if (scratch && prefill_tile_takes(seq, n_heads, hd) && prefill_tile_aligned(q, k))
     return launch_prefill_tile(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, aq, quantized, s);
   return launch_attn<false>(q, k, v, 0, nullptr, seq, n_heads, n_kv_heads, hd, out, scratch, seq, aq, quantized, 0, s);
 }

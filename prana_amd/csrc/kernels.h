@@ -245,7 +245,7 @@ int launch_attention_cache(const float* q, const uint16_t* kc, const uint16_t* v
 // Score scratch a launch needs: cache windows keep the scores of every (query
 // row, head) there on the split path; probabilities beyond 4096 positions
 // spill from LDS to it on the one-launch path; a prefill on the tiled kernel
-// (aligned: q, k and v on 16 bytes) keeps its workgroups' score rows there.
+// (aligned: q and k on 16 bytes) keeps its workgroups' score rows there.
 // Also the dim slices per head a launch uses.
 size_t attention_scratch_floats(size_t n_q, size_t n_heads, size_t ctx_cap);
 size_t attention_prefill_scratch_floats(size_t seq, size_t n_heads, size_t hd, bool aligned);
@@ -257,14 +257,14 @@ int launch_attention_prefill(const float* q, const float* k, const float* v, siz
                              const ActQuant* aq = nullptr, bool* quantized = nullptr);
 
 // ---- prefill_attention.hip
-// The tiled prefill attention: 16-byte aligned q, k and v
+// The tiled prefill attention: 16-byte aligned q and k
 // (prefill_tile_aligned), head widths that are multiples of 4 up to 256, and
 // enough query rows (prefill_tile_takes).
 // scratch >= prefill_tile_scratch_floats(seq, n_heads, hd) floats: the rows of
 // the launch's slots.
 size_t prefill_tile_scratch_floats(size_t seq, size_t n_heads, size_t hd);
 bool prefill_tile_takes(size_t seq, size_t n_heads, size_t hd);
-bool prefill_tile_aligned(const float* q, const float* k, const float* v);
+bool prefill_tile_aligned(const float* q, const float* k);
 int launch_prefill_tile(const float* q, const float* k, const float* v, size_t seq, size_t n_heads,
                         size_t n_kv_heads, size_t hd, float* out, float* scratch, const ActQuant* aq,
                         bool* quantized, hipStream_t s);

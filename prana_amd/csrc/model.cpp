@@ -251,7 +251,7 @@ int Model::ensure_ws(size_t n_tok, size_t ctx_cap, bool prefill_attn) {
     PRANA_HIP(hipMemset(ws.xch.p, 0, ws.xch.bytes));
     ws.gen++;
   }
-  // (the workspace's q, k and v are allocations: aligned)
+  // (the workspace's q and k are allocations: aligned)
   size_t need = (prefill_attn ? attention_prefill_scratch_floats(n_tok, c.n_heads, c.head_dim, true)
                               : attention_scratch_floats(n_tok, c.n_heads, ctx_cap)) * 4;
   const void* before = ws.scratch.p;

@@ -2,11 +2,14 @@
 `attention` (attention.rs:236-284), bit for bit: block and tile edges (16 / 32 / 64
 query rows, 128 / 256 keys), head widths that fill a lane tile or leave part
 of it empty, several blocks per workgroup, and non-finite K and V rows."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import prana_amd as P
 from oracle import oracle as O
+from prana_amd import check, load
 
 pytestmark = pytest.mark.gpu
 
@@ -33,6 +36,19 @@ def qkv(seq, nh, nkv, hd):
 def test_prefill_tile(seq, nh, nkv, hd):
     q, k, v = qkv(seq, nh, nkv, hd)
     assert same_bits(P.attention_prefill(q, k, v, seq, nh, nkv, hd), O.attention(q, k, v, seq, nh, nkv, hd))
+
+
+# v at any f32 address runs the same kernel as an aligned one (its slots of
+# scratch), with the same bits; q or k off 16 bytes runs the one-launch kernel
+@pytest.mark.parametrize("seq,nh,nkv,hd", [(350, 6, 2, 128), (320, 128, 16, 64), (129, 8, 1, 20), (300, 4, 1, 132)])
+@pytest.mark.parametrize("shift", [(0, 0, 1), (0, 0, 2), (0, 0, 3), (1, 0, 0), (0, 3, 0)])
+def test_prefill_unaligned(seq, nh, nkv, hd, shift):
+    host = qkv(seq, nh, nkv, hd)
+    d = [P.DeviceArray.from_host(np.concatenate([np.zeros(s, np.float32), a])) for s, a in zip(shift, host)]
+    out = P.DeviceArray((seq * nh * hd,), np.float32)
+    check(load().prana_attention_prefill(*[C.c_void_p(a.ptr.value + 4 * s) for s, a in zip(shift, d)], seq, nh, nkv,
+                                         hd, out.ptr, None))
+    assert same_bits(out.to_host(), O.attention(*host, seq, nh, nkv, hd).ravel())
 
 
 def test_prefill_tile_nonfinite():
