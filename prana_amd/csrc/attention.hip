@@ -1101,6 +1101,220 @@ int launch_wide(const float* q, const uint16_t* k, const uint16_t* v, size_t pos
   return kOk;
 }
 
+// ---------------------------------------------------------------- prefill blocks
+// Prefill attention over the f32 K/V of the window (attention.rs:236-284)
+// with one 256-lane workgroup per (head, pair of blocks of kPbQ consecutive
+// query rows, one from each end of the causal window, taken one after the
+// other): each K row a lane fetches serves the block's kPbQ score chains (side
+// by side), and each V element a lane fetches serves kPbQ*hd/256 P·V chains.
+// Row qq of the block attends keys 0..i0+qq; its softmax sum is the exact
+// left-to-right fold, one row after another. Bound by latency (row-per-lane K
+// gathers, the sums); the short blocks and the pairing suit launches that
+// leave the chip part empty (prefill_blk_takes).
+constexpr int kPbQ = 8;
+constexpr int kPbNT = 256;
+constexpr int kPbMax = 2048;  // window rows a block workgroup takes
+constexpr int kPbW = exact::run_pad(kPbMax - 1) + 1;
+
+// DYN: the probability rows are dynamic LDS of scw words each (windows up to
+// kPbDynMax: several workgroups per CU); otherwise a static array sized for
+// kPbMax positions (the compiler then keeps more of the score loop in
+// registers, which long windows need more than occupancy).
+constexpr size_t kPbDynMax = 1024;
+template <int HD, bool DYN>
+__global__ __launch_bounds__(kPbNT) void attn_prefill_blk(const float* __restrict__ q, const float* __restrict__ k,
+                                                          const float* __restrict__ v, int seq, int n_heads,
+                                                          int group, float* __restrict__ out,
+                                                          int8_t* __restrict__ qd, float* __restrict__ qsa,
+                                                          int* __restrict__ qsum, int scw_arg) {
+  static_assert(HD % 4 == 0 && (kPbQ * HD) % kPbNT == 0, "whole chains per lane");
+  constexpr int QPL = kPbQ * HD / kPbNT;  // P·V chains per lane
+  constexpr int QSTEP = kPbNT / HD;       // query rows between a lane's chains
+  __shared__ __align__(16) float s_q[kPbQ][HD];
+  // the block's probability rows, scw words each (run_pad layout)
+  __shared__ __align__(16) float s_sc_st[DYN ? 4 : kPbQ * kPbW];
+  extern __shared__ float4 pb_smem[];
+  float* s_scd = DYN ? reinterpret_cast<float*>(pb_smem) : s_sc_st;
+  const int scw = DYN ? scw_arg : kPbW;
+  __shared__ float s_red[kPbQ][kPbNT / 64];
+  const int h = blockIdx.x, tid = threadIdx.x;
+  // Workgroup y takes query blocks y and nqb-1-y (the causal window's short
+  // and long ends), so every workgroup has about the same keys to cover
+  const int nqb = (seq + kPbQ - 1) / kPbQ;
+  for (int pass = 0; pass < 2; pass++) {
+    const int qb = pass == 0 ? static_cast<int>(blockIdx.y) : nqb - 1 - static_cast<int>(blockIdx.y);
+    if (pass == 1) {
+      if (qb <= static_cast<int>(blockIdx.y)) break;  // uniform: an odd count's middle block, done once
+      __syncthreads();  // the first block's reads of the LDS rows are done
+    }
+    const int i0 = qb * kPbQ;
+    const int nk = min(i0 + kPbQ, seq);  // keys any row of the block attends
+    const int kvh = h / group;
+    const int kv_dim = (n_heads / group) * HD;
+    for (int e = tid; e < kPbQ * HD; e += kPbNT) {
+      const int qq = e / HD, d = e % HD;
+      s_q[qq][d] = i0 + qq < seq ? q[((size_t)(i0 + qq) * n_heads + h) * HD + d] : 0.0f;
+    }
+    __syncthreads();
+    // ---- scores: (fold_d q[d]*k_t[d] from -0.0) * (1/sqrt(hd)), lane per key row
+    const float scale = 1.0f / sqrtf(static_cast<float>(HD));
+    float mxl[kPbQ];
+#pragma unroll
+    for (int qq = 0; qq < kPbQ; qq++) mxl[qq] = -INFINITY;
+    for (int t = tid; t < nk; t += kPbNT) {
+      const float4* kp = reinterpret_cast<const float4*>(k + (size_t)t * kv_dim + (size_t)kvh * HD);
+      float dot[kPbQ];
+#pragma unroll
+      for (int qq = 0; qq < kPbQ; qq++) dot[qq] = -0.0f;
+#pragma unroll 4
+      for (int c = 0; c < HD / 4; c++) {
+        const float4 kv = kp[c];
+#pragma unroll
+        for (int qq = 0; qq < kPbQ; qq++) {
+          const float4 qv = reinterpret_cast<const float4*>(s_q[qq])[c];
+          dot[qq] += qv.x * kv.x;
+          dot[qq] += qv.y * kv.y;
+          dot[qq] += qv.z * kv.z;
+          dot[qq] += qv.w * kv.w;
+        }
+      }
+#pragma unroll
+      for (int qq = 0; qq < kPbQ; qq++) {
+        if (t <= i0 + qq) {  // causal: row i0+qq attends keys 0..i0+qq
+          const float sv = dot[qq] * scale;
+          s_scd[(qq) * scw + exact::run_pad(t)] = sv;
+          mxl[qq] = fmaxf(mxl[qq], sv);
+        }
+      }
+    }
+#pragma unroll
+    for (int qq = 0; qq < kPbQ; qq++) {
+      const float m = wave_max_f32(mxl[qq]);
+      if ((tid & 63) == 0) s_red[qq][tid >> 6] = m;
+    }
+    __syncthreads();
+    float mx[kPbQ];
+#pragma unroll
+    for (int qq = 0; qq < kPbQ; qq++) {
+      mx[qq] = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < kPbNT / 64; w++) mx[qq] = fmaxf(mx[qq], s_red[qq][w]);
+    }
+#pragma unroll
+    for (int qq = 0; qq < kPbQ; qq++) {
+      const int n = i0 + qq + 1;
+      if (i0 + qq < seq)
+        for (int t = tid; t < n; t += kPbNT) s_scd[(qq) * scw + exact::run_pad(t)] = dev_expf(s_scd[(qq) * scw + exact::run_pad(t)] - mx[qq]);
+    }
+    __syncthreads();
+    // softmax sums in the reference's left-to-right order (norms.rs:53): each
+    // wave folds one row at a time, the waves' rows at once
+    __shared__ float s_inv[kPbQ];
+    static_assert(kPbQ % (kPbNT / 64) == 0, "whole rounds of rows");
+#pragma unroll
+    for (int r = 0; r < kPbQ / (kPbNT / 64); r++) {
+      const int qq = r * (kPbNT / 64) + (tid >> 6);
+      if (i0 + qq < seq) {  // wave-uniform; the group barriers are the wave's own
+        const float sum =
+            exact::group_seq_sum_short<64, kPbNT / 64>([s_scd, scw, qq](int t) { return s_scd[(qq) * scw + exact::run_pad(t)]; }, i0 + qq + 1);
+        if ((tid & 63) == 0) s_inv[qq] = sum > 0.0f ? 1.0f / sum : 0.0f;
+      } else if ((tid & 63) == 0) {
+        s_inv[qq] = 0.0f;
+      }
+    }
+    __syncthreads();
+    float inv[kPbQ];
+#pragma unroll
+    for (int qq = 0; qq < kPbQ; qq++) inv[qq] = s_inv[qq];
+#pragma unroll
+    for (int qq = 0; qq < kPbQ; qq++) {
+      const int n = i0 + qq + 1;
+      if (i0 + qq < seq)
+        for (int t = tid; t < n; t += kPbNT) s_scd[(qq) * scw + exact::run_pad(t)] = s_scd[(qq) * scw + exact::run_pad(t)] * inv[qq];
+    }
+    __syncthreads();
+    // ---- P·V: lane (d, qg) folds rows qg, qg+QSTEP, ... of dim d over t from +0.0
+    const int d = tid % HD, qg = tid / HD;
+    const float* vcol = v + (size_t)kvh * HD + d;
+    float acc[QPL];
+#pragma unroll
+    for (int c = 0; c < QPL; c++) acc[c] = 0.0f;
+    // rows 0..i0 are attended by every query row of the block: no causal test
+    // there, so the probability and V reads of a batch issue together; only
+    // the last kPbQ - 1 keys need the per-row select
+    int t = 0;
+    for (; t + 8 <= i0 + 1; t += 8) {
+      float vt[8], pt[8][QPL];
+#pragma unroll
+      for (int u = 0; u < 8; u++) vt[u] = vcol[(size_t)(t + u) * kv_dim];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+#pragma unroll
+        for (int c = 0; c < QPL; c++) pt[u][c] = s_scd[(qg + c * QSTEP) * scw + exact::run_pad(t + u)];
+#pragma unroll
+      for (int u = 0; u < 8; u++)
+#pragma unroll
+        for (int c = 0; c < QPL; c++) acc[c] = acc[c] + pt[u][c] * vt[u];
+    }
+    for (; t <= i0; t++) {
+      const float vt = vcol[(size_t)t * kv_dim];
+#pragma unroll
+      for (int c = 0; c < QPL; c++) acc[c] = acc[c] + s_scd[(qg + c * QSTEP) * scw + exact::run_pad(t)] * vt;
+    }
+    for (; t < nk; t++) {
+      const float vt = vcol[(size_t)t * kv_dim];
+#pragma unroll
+      for (int c = 0; c < QPL; c++) {
+        const int qq = qg + c * QSTEP;
+        const float nv = acc[c] + s_scd[(qq) * scw + exact::run_pad(t)] * vt;
+        acc[c] = t <= i0 + qq ? nv : acc[c];
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < QPL; c++) {
+      const int qq = qg + c * QSTEP, i = i0 + qq;
+      const bool live = i < seq;
+      const size_t gi = ((size_t)min(i, seq - 1) * n_heads + h) * HD + d;
+      if (live) out[gi] = acc[c];
+      if (qd) {  // 32-lane groups share qq (HD is a multiple of 32 here)
+        float qscale;
+        int qs;
+        const int qi = quantize_lane(live ? acc[c] : 0.0f, &qscale, &qs);
+        if (live) {
+          qd[gi] = static_cast<int8_t>(qi);
+          if ((gi & 31) == 0) {
+            qsa[gi >> 5] = qscale;
+            qsum[gi >> 5] = qs;
+          }
+        }
+      }
+    }
+  }
+}
+
+template <int HD>
+int launch_prefill_blk(const float* q, const float* k, const float* v, size_t seq, size_t n_heads,
+                       size_t n_kv_heads, float* out, const ActQuant* aq, bool* quantized, hipStream_t s) {
+  const bool fuse_q = aq && aq->q;
+  if (quantized) *quantized = fuse_q;
+  const size_t nqb = (seq + kPbQ - 1) / kPbQ;
+  const dim3 grid(n_heads, (nqb + 1) / 2);  // a pair of query blocks per workgroup
+  int8_t* qd = fuse_q ? aq->q : nullptr;
+  float* qsa = fuse_q ? aq->sa : nullptr;
+  int* qsum = fuse_q ? aq->sums : nullptr;
+  const int group = static_cast<int>(n_heads / n_kv_heads);
+  if (seq <= kPbDynMax) {
+    const int scw = (exact::run_pad(static_cast<int>(seq) - 1) + 1 + 3) & ~3;  // 16-byte aligned rows
+    hipLaunchKernelGGL((attn_prefill_blk<HD, true>), grid, dim3(kPbNT), (size_t)kPbQ * scw * sizeof(float), s, q, k,
+                       v, (int)seq, (int)n_heads, group, out, qd, qsa, qsum, scw);
+  } else {
+    hipLaunchKernelGGL((attn_prefill_blk<HD, false>), grid, dim3(kPbNT), 0, s, q, k, v, (int)seq, (int)n_heads,
+                       group, out, qd, qsa, qsum, 0);
+  }
+  PRANA_LAUNCH_CHECK();
+  return kOk;
+}
+
 // grid: (n_heads*dsplit, n_q). Query row i sits at position p0 + i.
 // mode: 0 scalar rows; -1 vector V chunks with a runtime head width;
 // 48/64/128 vector K and V loads with that compiled head width.
@@ -1297,10 +1511,26 @@ size_t attention_scratch_floats(size_t n_q, size_t n_heads, size_t ctx_cap) {
   return std::max(n_q * n_heads * split_stride(ctx_cap), spill_floats(n_q, n_heads, ctx_cap));
 }
 
+// Few heads over a long window: the tiled kernel's 16-row blocks give at most
+// two workgroups per compute unit, and its longest block alone sets the time.
+// 8-row blocks in pairs are faster from about 600 positions on for 128-wide
+// heads, and for 64-wide ones from 1025 on, where they have static LDS rows: 1
+// head x 64 at 1150 positions 95 against 111 us and at 2048 137 against 175, 4
+// x 64 at 1500 121 against 136; 2 x 128 at 2048 188 against 308, 4 x 128 at
+// 699 115 against 126, 8 x 128 at 1024 146 against 164. Shorter windows
+// and more heads are the tiled kernel's (4 x 64 at 1024 101 against 96, 8 x 128
+// at 570 111 against 107, 6 x 64 at 1500 206 against 137), and one 128-wide
+// head below 950 positions the one-launch kernel's (850: 130 against 118).
+static bool prefill_blk_takes(size_t seq, size_t n_heads, size_t hd) {
+  return (hd == 64 || hd == 128) && seq <= static_cast<size_t>(kPbMax) && seq >= (hd == 64 ? kPbDynMax + 1 : 594) &&
+         seq * n_heads >= 950 && (seq + 15) / 16 * n_heads <= 512;
+}
+
 // Sized by the kernel that takes the shape: a long prompt on the tiled kernel
 // needs its slots only (32 heads x 16384 positions 3.2 GB), not the one-launch
 // kernel's score rows (34 GB).
 size_t attention_prefill_scratch_floats(size_t seq, size_t n_heads, size_t hd, bool aligned) {
+  if (aligned && prefill_blk_takes(seq, n_heads, hd)) return 0;
   if (aligned && prefill_tile_takes(seq, n_heads, hd)) return prefill_tile_scratch_floats(seq, n_heads, hd);
   return spill_floats(seq, n_heads, seq);
 }
@@ -1323,7 +1553,11 @@ int launch_attention_prefill(const float* q, const float* k, const float* v, siz
   if (seq == 0) return kOk;
   PRANA_CHECK(n_kv_heads > 0 && n_heads % n_kv_heads == 0, "attention: n_heads must be a multiple of n_kv_heads");
   PRANA_CHECK(hd > 0 && hd <= 256, "attention: head_dim must be in 1..=256");
-  if (scratch && prefill_tile_takes(seq, n_heads, hd) && prefill_tile_aligned(q, k))
+  const bool aligned = prefill_tile_aligned(q, k);
+  if (aligned && prefill_blk_takes(seq, n_heads, hd))
+    return hd == 64 ? launch_prefill_blk<64>(q, k, v, seq, n_heads, n_kv_heads, out, aq, quantized, s)
+                    : launch_prefill_blk<128>(q, k, v, seq, n_heads, n_kv_heads, out, aq, quantized, s);
+  if (scratch && aligned && prefill_tile_takes(seq, n_heads, hd))
     return launch_prefill_tile(q, k, v, seq, n_heads, n_kv_heads, hd, out, scratch, aq, quantized, s);
   return launch_attn<false>(q, k, v, 0, nullptr, seq, n_heads, n_kv_heads, hd, out, scratch, seq, aq, quantized, 0, s);
 }

@@ -38,9 +38,22 @@ def test_prefill_tile(seq, nh, nkv, hd):
     assert same_bits(P.attention_prefill(q, k, v, seq, nh, nkv, hd), O.attention(q, k, v, seq, nh, nkv, hd))
 
 
+# few heads over windows of up to 2048 positions: pairs of 8-row blocks
+# (attention.hip), the middle block of an odd count taken once, a part block at
+# the end; the first and last window of each width's range, and the tiled
+# kernel on the other side of each line
+@pytest.mark.parametrize("seq,nh,nkv,hd", [
+    (950, 1, 1, 128), (949, 1, 1, 128), (594, 2, 1, 128), (593, 2, 1, 128), (699, 4, 2, 128), (1024, 8, 8, 128), (1025, 3, 1, 128), (2048, 4, 2, 128),
+    (1025, 1, 1, 64), (1024, 2, 1, 64), (1500, 4, 2, 64), (2041, 3, 3, 64), (2048, 4, 1, 64), (2049, 2, 2, 64),
+    (1200, 7, 7, 64)])
+def test_prefill_few_heads(seq, nh, nkv, hd):
+    test_prefill_tile(seq, nh, nkv, hd)
+
+
 # v at any f32 address runs the same kernel as an aligned one (its slots of
 # scratch), with the same bits; q or k off 16 bytes runs the one-launch kernel
-@pytest.mark.parametrize("seq,nh,nkv,hd", [(350, 6, 2, 128), (320, 128, 16, 64), (129, 8, 1, 20), (300, 4, 1, 132)])
+@pytest.mark.parametrize("seq,nh,nkv,hd", [(350, 6, 2, 128), (320, 128, 16, 64), (129, 8, 1, 20), (300, 4, 1, 132),
+                                            (1200, 2, 1, 64)])
 @pytest.mark.parametrize("shift", [(0, 0, 1), (0, 0, 2), (0, 0, 3), (1, 0, 0), (0, 3, 0)])
 def test_prefill_unaligned(seq, nh, nkv, hd, shift):
     host = qkv(seq, nh, nkv, hd)
