@@ -452,11 +452,24 @@ size_t prefill_tile_scratch_floats(size_t seq, size_t n_heads, size_t hd) {
 }
 
 // Below these (query row, head) counts the one-launch kernel's workgroup per
-// row and head is faster: 14 heads x 32 positions 21 against 26 us, 6 x 100
-// 26 against 28, 16 x 50 32 against 29, 32 x 32 34 against 31; 256-wide
-// heads, 8 x 120 61 against 67, 8 x 300 211 against 111.
+// row and head is faster. Its time grows with rows x positions x head width,
+// the tiled kernel's with positions and the padded width, so the line falls
+// with more heads and with a fuller padded width: 1 head x 16 at 1500 positions
+// 77 against 96 us, at 2600 166 against 157; 1 x 48 at 1000 72 against 87; 2 x
+// 80 at 600 75 against 96; 4 x 128 at 250 56 against 55; 16 x 96 at 44 28
+// against 28; 256-wide heads, 8 x 120 61 against 67, 8 x 300 211 against 111.
+static size_t pt_min_rows(size_t n_heads, size_t hd) {
+  static const unsigned rows[4][5] = {// heads 1, 2, 3-5, 6-15, 16 and more
+                                      {2100, 1450, 1050, 750, 700},    // up to 32 dims
+                                      {1400, 1220, 1080, 1040, 700},   // 64
+                                      {1800, 1600, 1400, 1080, 840},   // 112
+                                      {1250, 1200, 1180, 1080, 900}};  // 128
+  if (hd > 128) return 1100;
+  return rows[hd <= 32 ? 0 : hd <= 64 ? 1 : hd <= 112 ? 2 : 3]
+             [n_heads < 3 ? n_heads - 1 : n_heads < 6 ? 2 : n_heads < 16 ? 3 : 4];
+}
 bool prefill_tile_takes(size_t seq, size_t n_heads, size_t hd) {
-  return hd % 4 == 0 && hd <= 256 && seq >= 16 && seq * n_heads >= (hd <= 128 ? 700u : 1100u) &&
+  return hd % 4 == 0 && hd <= 256 && seq >= 16 && n_heads > 0 && seq * n_heads >= pt_min_rows(n_heads, hd) &&
          seq <= static_cast<size_t>(INT32_MAX) / 2;
 }
 // (v may sit at any f32 address: 14 heads x 64 at 2048 positions take the one-launch

@@ -38,6 +38,15 @@ def test_prefill_tile(seq, nh, nkv, hd):
     assert same_bits(P.attention_prefill(q, k, v, seq, nh, nkv, hd), O.attention(q, k, v, seq, nh, nkv, hd))
 
 
+# both sides of the row count from which a shape takes the tiled kernel
+@pytest.mark.parametrize("seq,nh,nkv,hd", [
+    (2099, 1, 1, 32), (2100, 1, 1, 32), (725, 2, 1, 16), (724, 2, 1, 16), (58, 18, 6, 48), (57, 18, 6, 48),
+    (400, 4, 1, 36), (260, 4, 4, 64), (280, 5, 5, 80), (279, 5, 5, 80), (255, 6, 2, 96), (180, 6, 1, 112), (179, 6, 1, 112),
+    (180, 6, 2, 128), (179, 6, 2, 128), (138, 8, 8, 256), (137, 8, 8, 256)])
+def test_prefill_line(seq, nh, nkv, hd):
+    test_prefill_tile(seq, nh, nkv, hd)
+
+
 # few heads over windows of up to 2048 positions: pairs of 8-row blocks
 # (attention.hip), the middle block of an odd count taken once, a part block at
 # the end; the first and last window of each width's range, and the tiled
