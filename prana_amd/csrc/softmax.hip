@@ -35,8 +35,6 @@ namespace prana {
 namespace {
 
 // ---------------------------------------------------------------- short rows
-// One workgroup per row; the sum is the sequential fold, evaluated exactly by
-// the workgroup.
 // norms.rs:44-56, one workgroup per row; the sum is the sequential fold,
 // evaluated exactly by the workgroup.
 __global__ __launch_bounds__(256) void softmax_kernel(const float* __restrict__ in, int n, float* __restrict__ out) {
@@ -391,9 +389,19 @@ __global__ __launch_bounds__(kSmNT) void softmax_scale_kernel(const float* in, f
   }
 }
 
-// One row of 8000 values 18 against 31 us, 75 rows of 8000 31 against 36, 100
-// rows of 6000 30 against 28.
-constexpr size_t kSmLongMin = 7168;
+// Rows of n values that the chunked launches take at most. They read the input
+// five times and evaluate each exponential three times, so many rows, which
+// fill the chip on one workgroup each, are the short kernel's: 64 rows of 8000
+// 31 (chunked) against 36 us, 256 rows 43 against 36; 192 rows of 11000 0.94
+// of its time, 256 1.14; 768 rows of 12000 0.96, 2048 1.15; 1 row of 7168 18
+// against 24 us. From 13000 values on all rows are chunked: 1024 rows 0.95-0.98,
+// 2048 1.05-1.14, 3000 0.89-0.96, and the short kernel folds a row whose
+// predicted scan fails, or of more than 16416 values, in a pass per binade (1024
+// rows of 16400 152 against 1130 us, of 32000 265 against 2434).
+size_t long_rows(size_t n) {
+  if (n < 7168) return 0;
+  return n < 8000 ? 64 : n < 10000 ? 96 : n < 12000 ? 192 : n < 13000 ? 768 : 65535;
+}
 
 }  // namespace
 
@@ -401,7 +409,7 @@ int launch_softmax(const float* in, size_t rows, size_t n, float* out, hipStream
   if (rows == 0 || n == 0) return kOk;
   const float *in1 = in + rows * n, *out1 = out + rows * n;
   const bool overlap = in < out1 && out < in1;
-  if (n < kSmLongMin || n > static_cast<size_t>(INT_MAX) / 2 || overlap || rows > 65535) {
+  if (rows > long_rows(n) || n > static_cast<size_t>(INT_MAX) / 2 || overlap) {
     hipLaunchKernelGGL(softmax_kernel, dim3(rows), dim3(256), 0, s, in, (int)n, out);
     PRANA_LAUNCH_CHECK();
     return kOk;

@@ -48,6 +48,19 @@ def test_softmax_long(kind, rows, n):
         assert same(got[i], O.softmax(x[i])), (kind, i)
 
 
+# the last row count of each range on the chunked launches, and the next one on
+# a workgroup per row
+@pytest.mark.parametrize("rows,n", [(64, 7168), (65, 7999), (96, 8000), (97, 9999), (192, 10000), (193, 11999),
+                                    (768, 12000), (769, 12999), (769, 13000)])
+def test_softmax_row_counts(rows, n):
+    x = rows_like("normal", rows, n)
+    x[rows // 2] = rows_like("ramp", 1, n)
+    got = P.softmax(x)
+    for i in (0, 1, rows // 2, rows - 2, rows - 1):
+        assert same(got[i], O.softmax(x[i])), i
+    assert np.all(np.abs(got.sum(1, dtype=np.float64) - 1) < 1e-4)  # every row was written (the 32-bit sum drifts by < 3e-9 n)
+
+
 def test_softmax_long_many_rows_and_past_2_24():
     x = rows_like("normal", 70, 7500)
     got = P.softmax(x)
