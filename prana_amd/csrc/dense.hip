@@ -2,10 +2,10 @@
 // row). Four strided partial sums (class l adds x[4i+l]*w[4i+l] over i from
 // 0.0, products and sums rounded separately), combined ((a0+a1)+a2)+a3, then
 // the tail of cols % 4 elements. The four classes are independent chains, so
-// both kernels keep them in separate lanes, and stage x and w in LDS class by
-// class: four consecutive terms of a chain are one 16-byte read. Chunks are
-// zero-padded past cols/4: adding +0.0 leaves a chain (started from +0.0)
-// unchanged.
+// the kernels keep them in separate lanes. Those for a few tokens and for
+// batches stage x and w in LDS class by class: four consecutive terms of a
+// chain are one 16-byte read. Chunks are zero-padded past cols/4: adding +0.0
+// leaves a chain (started from +0.0) unchanged.
 #include "common.h"
 #include "kernels.h"
 
@@ -37,6 +37,49 @@ __device__ __forceinline__ f4 load_quad(const float* row, int i, int nq) {
     v = f4{row[4 * j], row[4 * j + 1], row[4 * j + 2], row[4 * j + 3]};
   }
   return i < nq ? v : f4{0, 0, 0, 0};
+}
+
+// ---------------------------------------------------------------- narrow rows
+// One lane per class and row, operands read from memory (a row is a cache line
+// or a few): no staging to wait for. Bound by launch and load latency.
+__global__ __launch_bounds__(256) void gemv_f32_narrow_kernel(const float* __restrict__ w, int rows, int cols,
+                                                              const float* __restrict__ x, GemvOut o) {
+  __shared__ float part[256];
+  const int tok = blockIdx.y, l = threadIdx.x & 3;
+  const size_t r = (size_t)blockIdx.x * 64 + (threadIdx.x >> 2);
+  const float* xr = x + (size_t)tok * cols;
+  const float* wr = w + r * cols;
+  float acc = 0.0f;
+  if (r < static_cast<size_t>(rows))
+    for (int i = 0; i < cols / 4; i++) acc += xr[i * 4 + l] * wr[i * 4 + l];
+  part[threadIdx.x] = acc;
+  __syncthreads();
+  if (l == 0 && r < static_cast<size_t>(rows)) {
+    float sum = part[threadIdx.x] + part[threadIdx.x + 1] + part[threadIdx.x + 2] + part[threadIdx.x + 3];
+    for (int i = cols / 4 * 4; i < cols; i++) sum += xr[i] * wr[i];
+    store_dense(o, tok, r, sum);
+  }
+}
+
+// Short rows give the staging kernels one part-filled chunk and nothing to read
+// ahead, so little work is done sooner without it (staged against this
+// kernel): 32000 x 24 at one token 7.4 against 3.5 us, at 8 8.7 against 6.6, 4096 x
+// 17 at 20 4.8 against 3.6, 1000 x 40 at 300 10.4 against 6.8, and one token over
+// many rows up to 200 columns (32000 x 192 8.7 against 6.2, 256 9.2 against 8.9).
+// The line falls as rows leave the cache line (10000 x 24 at 40 6.2 against 9.4, x
+// 55 at 8 5.3 against 7.1); rows below four columns are staged by nothing
+// (32000 x 1 at 8 3.8 against 3.4, at 40 6.8 against 9.5).
+bool narrow_takes(size_t rows, size_t cols, size_t n_tok) {
+  if (n_tok == 1 && rows >= 16000 && cols <= (rows >= 24000 ? 200u : 140u)) return true;
+  if (n_tok == 2 && rows >= 16000 && rows <= 40000 && cols <= 110) return true;
+  const size_t most = cols < 4 ? (n_tok <= 16 ? 3600000 : 2000000)
+                      : cols <= 17 ? 26000000
+                      : cols <= 24 ? (n_tok <= 16 ? 15000000 : 9000000)
+                      : n_tok <= 4 ? 6000000
+                      : rows > 5000 ? 3200000
+                      : rows < 1000 ? 4000000
+                      : cols <= 56 ? 13500000 : 6000000;
+  return cols < 96 && n_tok <= 65535 && rows * n_tok * (cols + 4) <= most;
 }
 
 // ---------------------------------------------------------------- a few tokens
@@ -264,6 +307,11 @@ __global__ __launch_bounds__(kDmNT) void gemm_f32_kernel(const float* __restrict
 
 template <bool VEC>
 int launch_dense(const float* w, int rows, int cols, const float* x, int n_tok, const GemvOut& o, hipStream_t s) {
+  if (narrow_takes(rows, cols, n_tok)) {
+    hipLaunchKernelGGL(gemv_f32_narrow_kernel, dim3((rows + 63) / 64, n_tok), dim3(256), 0, s, w, rows, cols, x, o);
+    PRANA_LAUNCH_CHECK();
+    return kOk;
+  }
   const size_t rt = (rows + kDmRows - 1) / kDmRows;
   auto jobs = [&](size_t tt) { return rt * ((n_tok + tt - 1) / tt); };
   // Larger batches with few tiles run as groups of eight tokens (4096 x 4096

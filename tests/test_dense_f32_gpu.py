@@ -54,3 +54,35 @@ def test_dense_unaligned_activations_and_residual_zero_signs():
         nan = np.isnan(want[:k])
         assert np.array_equal(np.isnan(got), nan)
         assert same_bits(got[~nan], want[:k][~nan])
+
+
+def narrow(rows, cols, n):
+    """Whether a lane per class and row takes the call, without staging (narrow_takes)."""
+    if n == 1 and rows >= 16000 and cols <= (200 if rows >= 24000 else 140):
+        return True
+    if n == 2 and 16000 <= rows <= 40000 and cols <= 110:
+        return True
+    most = ((3600000 if n <= 16 else 2000000) if cols < 4 else 26000000 if cols <= 17
+            else (15000000 if n <= 16 else 9000000) if cols <= 24 else 6000000 if n <= 4 else 3200000 if rows > 5000 else 4000000 if rows < 1000
+            else 13500000 if cols <= 56 else 6000000)
+    return cols < 96 and rows * n * (cols + 4) <= most
+
+
+# narrow matrices over many rows, both sides of the line: last row groups part
+# filled, a tail of 1-3 columns and none, activations 4 bytes off
+@pytest.mark.parametrize("rows,cols,n,taken", [(24001, 200, 1, True), (24001, 201, 1, False), (16001, 110, 2, True),
+                                               (16001, 111, 2, False), (10007, 3, 28, True), (20011, 2, 33, False),
+                                               (9001, 17, 137, True), (9001, 17, 138, False), (33001, 24, 16, True),
+                                               (1003, 56, 224, True), (1003, 56, 225, False), (5001, 26, 21, True),
+                                               (5001, 26, 22, False), (1003, 95, 20, True), (1003, 96, 20, False)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_dense_narrow(rows, cols, n, taken, shift):
+    assert narrow(rows, cols, n) == taken
+    w, x = make(rows, cols, n)
+    w[rows // 2, 0], x[0, cols - 1] = -0.0, -0.0
+    raw = w.view(np.uint8)
+    buf = P.DeviceArray.from_host(np.concatenate([np.zeros(shift, np.float32), x.ravel()]))
+    out = P.DeviceArray((n, rows), np.float32)
+    m = P.Matrix(P.F32, rows, cols, raw)
+    check(load().prana_matmul(m.h, C.c_void_p(buf.ptr.value + 4 * shift), n, out.ptr, None))
+    assert same_bits(out.to_host(), O.Mat.from_ggml(P.F32, rows, cols, raw).apply(x))
