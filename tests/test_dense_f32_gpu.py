@@ -32,7 +32,7 @@ def test_dense_shapes(rows, cols, n):
     assert same_bits(P.Matrix(P.F32, rows, cols, raw).apply(x), O.Mat.from_ggml(P.F32, rows, cols, raw).apply(x))
 
 
-# 16-, 32- and 64-token tiles
+# groups of eight tokens (few tiles), and 32- and 64-token tiles of one chunk or two
 @pytest.mark.parametrize("rows,cols,n", [(640, 96, 67), (2049, 68, 481), (4100, 36, 515)])
 def test_dense_batches(rows, cols, n):
     test_dense_shapes(rows, cols, n)
@@ -80,6 +80,31 @@ def test_dense_narrow(rows, cols, n, taken, shift):
     assert narrow(rows, cols, n) == taken
     w, x = make(rows, cols, n)
     w[rows // 2, 0], x[0, cols - 1] = -0.0, -0.0
+    raw = w.view(np.uint8)
+    buf = P.DeviceArray.from_host(np.concatenate([np.zeros(shift, np.float32), x.ravel()]))
+    out = P.DeviceArray((n, rows), np.float32)
+    m = P.Matrix(P.F32, rows, cols, raw)
+    check(load().prana_matmul(m.h, C.c_void_p(buf.ptr.value + 4 * shift), n, out.ptr, None))
+    assert same_bits(out.to_host(), O.Mat.from_ggml(P.F32, rows, cols, raw).apply(x))
+
+
+def batch_tile(rows, n):
+    """Tokens per tile of the batch kernel, 0 where groups of eight tokens run instead (launch_dense)."""
+    jobs = lambda tt: -(-rows // 64) * -(-n // tt)  # (rows of 96 columns and more)
+    if n <= 16 or jobs(16) < 400:
+        return 0
+    return 64 if jobs(64) >= 512 else 32 if jobs(32) >= 512 else 16
+
+
+# every tile of the batch kernel over five and more chunks of 64 columns (both
+# staging buffers are reused): rows of any and of whole 16-byte words, with a
+# tail of 1-3 columns and without, and whole words 4 bytes off
+@pytest.mark.parametrize("rows,cols,n,tile", [(2048, 389, 301, 16), (2048, 388, 301, 16), (2049, 325, 481, 32),
+                                              (2049, 324, 481, 32), (4100, 323, 515, 64), (4100, 320, 515, 64)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_dense_batch_tiles(rows, cols, n, tile, shift):
+    assert batch_tile(rows, n) == tile
+    w, x = make(rows, cols, n)
     raw = w.view(np.uint8)
     buf = P.DeviceArray.from_host(np.concatenate([np.zeros(shift, np.float32), x.ravel()]))
     out = P.DeviceArray((n, rows), np.float32)
