@@ -10,6 +10,7 @@ import pytest
 import prana_amd as P
 from oracle import oracle as O
 from prana_amd import check, load
+from prana_amd import models as M
 
 pytestmark = pytest.mark.gpu
 
@@ -36,6 +37,17 @@ def qkv(seq, nh, nkv, hd):
 def test_prefill_tile(seq, nh, nkv, hd):
     q, k, v = qkv(seq, nh, nkv, hd)
     assert same_bits(P.attention_prefill(q, k, v, seq, nh, nkv, hd), O.attention(q, k, v, seq, nh, nkv, hd))
+
+
+def block_rows(seq, nh, hd):
+    """Query rows per block of the tiled kernel, and its workgroups per compute unit (pt_plan)."""
+    jobs = lambda bq: -(-seq // bq) * nh
+    bq = 64 if jobs(64) >= 1024 else 32 if jobs(32) >= 640 else 16
+    if bq == 64 and hd > 128:
+        bq = 32
+    if bq == 16:
+        return bq, 3
+    return bq, 3 if hd <= (64 if bq == 64 else 128) and jobs(bq) >= 1000 else 2
 
 
 # both sides of the row count from which a shape takes the tiled kernel
@@ -88,3 +100,40 @@ def test_prefill_tile_nonfinite():
     gn, wn = np.isnan(got), np.isnan(want)
     assert np.array_equal(gn, wn)  # NaN payloads are not part of the contract
     assert np.array_equal(got[~gn].view(np.uint32), want[~wn].view(np.uint32))
+
+
+@pytest.mark.parametrize("seq,nh,hd,rows", [(350, 64, 64, 32), (140, 256, 128, 32), (330, 64, 160, 32),
+                                             (193, 256, 64, 64), (193, 256, 128, 64)])
+def test_prefill_tile_nonfinite_larger_blocks(seq, nh, hd, rows):
+    assert block_rows(seq, nh, hd)[0] == rows
+    q, k, v = qkv(seq, nh, 1, hd)
+    v = v.reshape(seq, hd)
+    v[40, 3], v[70, 5], v[100, hd - 1] = np.inf, np.nan, -np.inf
+    k = k.reshape(seq, hd)
+    k[120] = np.nan
+    k[130, 0] = np.inf
+    got = P.attention_prefill(q, k, v, seq, nh, 1, hd)
+    want = O.attention(q, k.ravel(), v.ravel(), seq, nh, 1, hd)
+    gn, wn = np.isnan(got), np.isnan(want)
+    assert np.array_equal(gn, wn)
+    assert np.array_equal(got[~gn].view(np.uint32), want[~wn].view(np.uint32))
+
+
+# the int8 copy of the output that wo reads (head widths of whole 32-blocks),
+# from every block size, width and workgroup count: the second layer's K and V
+# rows hold what the first layer's attention gave
+@pytest.mark.parametrize("seq,nh,nkv,hd,plan", [
+    (100, 12, 4, 96, (16, 3)), (40, 64, 8, 128, (16, 3)), (50, 32, 4, 160, (16, 3)), (50, 32, 4, 224, (16, 3)),
+    (350, 64, 8, 64, (32, 2)), (70, 256, 16, 128, (32, 2)), (350, 96, 8, 96, (32, 3)), (140, 256, 16, 64, (32, 3)),
+    (129, 256, 16, 128, (32, 3)), (330, 64, 8, 160, (32, 2)), (321, 64, 4, 224, (32, 2)), (197, 160, 8, 256, (32, 2)),
+    (193, 256, 16, 32, (64, 3)), (193, 256, 16, 64, (64, 3)), (193, 256, 16, 128, (64, 2)), (200, 256, 8, 96, (64, 2))])
+def test_prefill_tile_quantized_output(seq, nh, nkv, hd, plan):
+    assert block_rows(seq, nh, hd) == plan
+    cfg = M.config(64, 96, 2, nh, nkv, 96, seq + 1, head_dim=hd)
+    t = M.synth_tensors(cfg, lambda name, cols: P.Q8_0, 5)
+    gc, oc = P.Model(cfg, t).cache(seq), O.Model(cfg, t).cache(seq)
+    prompt = np.random.default_rng(seq).integers(0, cfg["vocab_size"], seq).astype(np.uint32)
+    gc.prefill(prompt)
+    oc.prefill(prompt)
+    for which in (0, 1):
+        assert np.array_equal(gc.read(1, which, seq), oc.read(1, which, seq)), which
