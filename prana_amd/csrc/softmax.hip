@@ -2,7 +2,7 @@
 // the reference's left-to-right fold, e * (1/sum).
 //
 // Long rows (a vocabulary) are cut into chunks of about 1024 values, a
-// workgroup each, in five launches:
+// workgroup each, in five launches (seven from a million values on):
 //   1. each chunk's maximum
 //   2. each chunk's sum of exponentials, in any order
 //   3. each chunk's part of the ordered sum as a map: while the running sum
@@ -65,7 +65,9 @@ constexpr int kSmSlots = 16;             // chunks whose plain terms are fetched
 // row's maximum, launch 3 the maps (e0 o0 e1 o1), the plain additions and the
 // binades of the two runs (chunk 0: its exact sum, in kRecMap), launch 4 the
 // factor 1/sum.
-enum { kRecMax = 0, kRecSum = 1, kRecMap = 2, kRecPlain = 6, kRecB0 = 7, kRecB1 = 8, kRecInv = 9, kRecRowMax = 10 };
+enum {
+  kRecMax = 0, kRecSum = 1, kRecMap = 2, kRecPlain = 6, kRecB0 = 7, kRecB1 = 8, kRecInv = 9, kRecRowMax = 10, kRecPre = 11
+};
 constexpr int kComplex = 1 << 30;        // kRecPlain: no map, sum the chunk from the value before it
 
 // Chunk c of the row is [begin(c), begin(c + 1)): 512 values at least.
@@ -101,6 +103,49 @@ __global__ __launch_bounds__(kSmNT) void softmax_max_kernel(const float* in, flo
   if (threadIdx.x == 0) R.rec(c)[kRecMax] = mx;
 }
 
+// Rows of more than kSmMany chunks (about a million values): the row's maximum and the sums before each
+// chunk are formed by one workgroup per row, where otherwise every chunk's
+// workgroup reads the other chunks' records (work that grows with the square of
+// their number).
+constexpr int kSmScanNT = 1024;
+
+__global__ __launch_bounds__(kSmScanNT) void softmax_row_max_kernel(const float* in, float* out, int n, int chunks) {
+  __shared__ float s_red[kSmScanNT / 64];
+  const SmRow R = sm_row(in, out, n, chunks);
+  float mx = -INFINITY;
+  for (int c = threadIdx.x; c < chunks; c += kSmScanNT) mx = fmaxf(mx, R.rec(c)[kRecMax]);
+  mx = wave_max_f32(mx);
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kSmScanNT / 64; w++) mx = fmaxf(mx, s_red[w]);
+    R.out[kRecRowMax] = mx;
+  }
+}
+
+// kRecPre of every chunk: the sums before it, in any order.
+__global__ __launch_bounds__(kSmScanNT) void softmax_prefix_kernel(const float* in, float* out, int n, int chunks) {
+  __shared__ float s_wave[2][kSmScanNT / 64];
+  const SmRow R = sm_row(in, out, n, chunks);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float carry = 0.0f, next = tid < chunks ? R.rec(tid)[kRecSum] : 0.0f;
+  for (int c0 = 0, b = 0; c0 < chunks; c0 += kSmScanNT, b ^= 1) {
+    const int c = c0 + tid;
+    const float inc = exact::scan_add_f32(next);
+    next = c + kSmScanNT < chunks ? R.rec(c + kSmScanNT)[kRecSum] : 0.0f;
+    if (lane == 63) s_wave[b][wave] = inc;
+    __syncthreads();  // (the buffer of the pass before last is free again)
+    const float before = __int_as_float(exact::wave_shr1(__float_as_int(inc)));  // the lane before's, 0 in lane 0
+    float pre = carry;
+    for (int w = 0; w < kSmScanNT / 64; w++) {
+      if (w == wave && c < chunks) R.rec(c)[kRecPre] = pre + before;
+      pre += s_wave[b][w];
+    }
+    carry = pre;
+  }
+}
+
+template <bool MANY>  // the row's maximum is in the first record
 __global__ __launch_bounds__(kSmNT) void softmax_sum_kernel(const float* in, float* out, int n, int chunks) {
   __shared__ float s_red[kSmNT / 64], s_sum[kSmNT / 64];
   const SmRow R = sm_row(in, out, n, chunks);
@@ -108,8 +153,12 @@ __global__ __launch_bounds__(kSmNT) void softmax_sum_kernel(const float* in, flo
   float x[kSmCT], mx = -INFINITY;
 #pragma unroll
   for (int u = 0; u < kSmCT; u++) x[u] = R.in[min(b + tid + kSmNT * u, e - 1)];
-  for (int d = tid; d < chunks; d += kSmNT) mx = fmaxf(mx, R.rec(d)[kRecMax]);
-  mx = sm_block_max(mx, s_red);
+  if constexpr (MANY) {
+    mx = R.out[kRecRowMax];
+  } else {
+    for (int d = tid; d < chunks; d += kSmNT) mx = fmaxf(mx, R.rec(d)[kRecMax]);
+    mx = sm_block_max(mx, s_red);
+  }
   float s = 0.0f;
 #pragma unroll
   for (int u = 0; u < kSmCT; u++) {
@@ -122,7 +171,7 @@ __global__ __launch_bounds__(kSmNT) void softmax_sum_kernel(const float* in, flo
   __syncthreads();
   if (tid == 0) {
     R.rec(c)[kRecSum] = (s_sum[0] + s_sum[1]) + (s_sum[2] + s_sum[3]);
-    R.rec(c)[kRecRowMax] = mx;
+    if (!MANY || c > 0) R.rec(c)[kRecRowMax] = mx;
   }
 }
 
@@ -185,6 +234,7 @@ __device__ float sm_continue(float s, const float (&v)[kSmCT], int* s_wave, int*
   return s;
 }
 
+template <bool MANY>  // kRecPre holds the sums before the chunk
 __global__ __launch_bounds__(kSmNT) void softmax_map_kernel(const float* in, float* out, int n, int chunks) {
   __shared__ float s_red[kSmNT / 64], s_pre[kSmNT / 64], s_term[exact::run_pad(kSmChunk)];
   __shared__ int s_wave[2 * (kSmNT / 64)], s_p0, s_p1, s_b1;
@@ -203,9 +253,13 @@ __global__ __launch_bounds__(kSmNT) void softmax_map_kernel(const float* in, flo
   }
   // approximate sum before the chunk (any order), then before this lane
   float pre = 0.0f;
-  for (int d = tid; d < c; d += kSmNT) pre += R.rec(d)[kRecSum];
+  if constexpr (MANY) {
+    pre = tid == 0 ? R.rec(c)[kRecPre] : 0.0f;
+  } else {
+    for (int d = tid; d < c; d += kSmNT) pre += R.rec(d)[kRecSum];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) pre += __shfl_xor(pre, o, 64);
+    for (int o = 32; o > 0; o >>= 1) pre += __shfl_xor(pre, o, 64);
+  }
   const float inc = exact::scan_add_f32((v[0] + v[1]) + (v[2] + v[3]));
   if (lane == 63) s_pre[wave] = inc;
   if (lane == 0) s_red[wave] = pre;
@@ -389,6 +443,13 @@ __global__ __launch_bounds__(kSmNT) void softmax_scale_kernel(const float* in, f
   }
 }
 
+// Chunks from which a row has launches of its own for its maximum and the sums
+// before each chunk: 1 x 4M values 261 -> 199 us, 3 x 4M 491 -> 285, 1 x 17M 4.1 -> 2.5
+// ms, 1 x 67M 76 -> 40 ms (3554 on the one-workgroup kernel); with fewer the two
+// launches cost as much as they save (1 x 800000 56 against 59, 1 x 1000000 60
+// against 62, 3 x 1000000 87 against 82).
+constexpr int kSmMany = 1000;
+
 // Rows of n values that the chunked launches take at most. They read the input
 // five times and evaluate each exponential three times, so many rows, which
 // fill the chip on one workgroup each, are the short kernel's: 64 rows of 8000
@@ -418,8 +479,15 @@ int launch_softmax(const float* in, size_t rows, size_t n, float* out, hipStream
   const dim3 grid(chunks, rows), nt(kSmNT);
   const int ni = static_cast<int>(n), nc = static_cast<int>(chunks);
   hipLaunchKernelGGL(softmax_max_kernel, grid, nt, 0, s, in, out, ni, nc);
-  hipLaunchKernelGGL(softmax_sum_kernel, grid, nt, 0, s, in, out, ni, nc);
-  hipLaunchKernelGGL(softmax_map_kernel, grid, nt, 0, s, in, out, ni, nc);
+  if (nc > kSmMany) {
+    hipLaunchKernelGGL(softmax_row_max_kernel, dim3(1, rows), dim3(kSmScanNT), 0, s, in, out, ni, nc);
+    hipLaunchKernelGGL(softmax_sum_kernel<true>, grid, nt, 0, s, in, out, ni, nc);
+    hipLaunchKernelGGL(softmax_prefix_kernel, dim3(1, rows), dim3(kSmScanNT), 0, s, in, out, ni, nc);
+    hipLaunchKernelGGL(softmax_map_kernel<true>, grid, nt, 0, s, in, out, ni, nc);
+  } else {
+    hipLaunchKernelGGL(softmax_sum_kernel<false>, grid, nt, 0, s, in, out, ni, nc);
+    hipLaunchKernelGGL(softmax_map_kernel<false>, grid, nt, 0, s, in, out, ni, nc);
+  }
   hipLaunchKernelGGL(softmax_walk_kernel, dim3(1, rows), nt, 0, s, in, out, ni, nc);
   hipLaunchKernelGGL(softmax_scale_kernel, grid, nt, 0, s, in, out, ni, nc);
   PRANA_LAUNCH_CHECK();

@@ -69,6 +69,21 @@ def test_softmax_long_many_rows_and_past_2_24():
     assert same(P.softmax(flat)[0], O.softmax(flat))
 
 
+# 1000 and 1001 chunks: the row's maximum and the sums before each chunk from
+# every chunk's workgroup, and from launches of their own (a full and a part
+# round of 1024 chunks)
+@pytest.mark.parametrize("rows,n", [(1, 1024000), (2, 1024001), (1, 1048577), (2, 1100003)])
+@pytest.mark.parametrize("kind", ["normal", "peak", "late", "ramp", "wide", "nonfinite"])
+def test_softmax_many_chunks(kind, rows, n):
+    x = rows_like(kind, rows, n)
+    if kind == "nonfinite":
+        x[0, n // 2] = np.nan
+        x[-1, : n - 700] = -np.inf
+    got = P.softmax(x)
+    for i in range(rows):
+        assert same(got[i], O.softmax(x[i])), (kind, i)
+
+
 def test_softmax_long_nonfinite_and_in_place():
     x = rows_like("normal", 5, 9000)
     x[0, 4000] = np.nan
