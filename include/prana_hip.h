@@ -15,8 +15,12 @@
  *     matmul.rs:31-39, kquant.rs:166-169, attention.rs:138-143) come back as
  *     PRANA_ERR_INVALID instead of aborting; nothing throws across the ABI;
  *   - kernel entry points take DEVICE pointers and a stream (NULL = the
- *     library's stream) and are asynchronous; model entry points take host
- *     buffers and synchronise before returning.
+ *     library's stream) and are asynchronous, but for these, which wait for
+ *     their stream before returning: prana_matmul on quantized matrices and
+ *     prana_attention_decode / _verify / _prefill / _decode_splitk (their
+ *     scratch serves all callers), the rope calls (a table of the call's own)
+ *     and prana_sampler_sample (its token goes to the host);
+ *   - model entry points take host buffers and synchronise before returning.
  *
  * Numerics: results are bit-identical to the reference's scalar tier
  * (integer block dots exact, f32 folds in the reference's order).

@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kDvNT) void gemv_f32_kernel(const float* __restrict
 // tokens x 8 rows of it: TT/8 + 8 16-byte LDS reads feed TT*8 vector
 // operations. Chunks of 64 elements, loaded two ahead. Bound by the vector
 // ALU (two operations per product): 4096 x 4096 over 512 tokens runs at 47
-// Tops/s of the 65 that many independent chains reach on this card. 2048 x
+// Tops/s of the 65-68 that many independent chains reach on this card. 2048 x
 // 2048 over 301 tokens: 86 us, 706 with a lane per class and row reading both
 // operands from memory. Reading LDS further ahead (a full unroll of the
 // chunk, 220 registers) is faster with one workgroup per compute unit and

@@ -10,10 +10,11 @@
 //
 // One 256-lane workgroup takes one head's block of BQ consecutive query rows
 // through three phases:
-//   1. scores. Tiles of 8192/BQ keys, 8 rows x 4 keys per lane: twelve
-//      16-byte LDS reads (q rows broadcast) per 4 dims feed 256 vector
-//      operations. K is staged 16 KB at a time, one stage ahead. Scores go to
-//      the workgroup's slot of global scratch (they stay in the caches).
+//   1. scores. Tiles of 8192/BQ keys, 8 rows x 4 keys per lane (BQ = 16: 256
+//      keys, 4 rows x 4 keys): twelve 16-byte LDS reads (q rows broadcast) per 4
+//      dims feed 256 vector operations (16: eight and 128). K is staged 16 KB
+//      at a time, one stage ahead. Scores go to the workgroup's slot of
+//      global scratch (they stay in the caches).
 //   2. softmax. All lanes turn a tile's scores into exponentials (back to the
 //      slot, and to LDS); one wave then folds the previous tile's
 //      exponentials with one lane per query row, so the left-to-right sums of
@@ -29,9 +30,11 @@
 // Measured (one MI355X, one call): 14 heads x 64 dims at 2048 positions 275
 // us and at 3001 505 us, 32 heads x 128 at 2048 963 us; the kernels before
 // took 550 (eight query rows per workgroup, one key row gathered per lane),
-// 5590 and 1760. At 32 x 128 x 2048 the counters show the vector ALU issuing
-// in every cycle, 17 % of its instructions not products or sums of the two
-// contractions (the causal diagonal, exponentials, addresses).
+// 5590 and 1760. At 32 x 128 x 2048 the counters show 1.09 vector instructions
+// per SIMD and four cycles (two waves can issue together; a probe of
+// independent operations reaches 1.9), 15 % of them not products or sums of
+// the two contractions (the causal diagonal, exponentials, addresses), and
+// waves waiting for memory and barriers 31 % of their time.
 #include <algorithm>
 
 #include "common.h"

@@ -21,7 +21,7 @@
 // the path needs no scratch and its launches keep nothing between calls; the
 // exponentials are recomputed from `in` where they are needed, so in and out
 // must not overlap. Bound by the latency of the five launches and the walk:
-// one row of 151936 values 26 us, of 32000 21 us, against 3790 and 744 us on
+// one row of 151936 values 26-27 us, of 32000 21 us, against 3845 and 744 us on
 // the one-workgroup kernel (an ordered pass of 256 lanes per binade); walking
 // the 149 records one by one took 36 of then 48 us.
 #include <climits>
