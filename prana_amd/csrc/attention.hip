@@ -1526,6 +1526,8 @@ static bool prefill_blk_takes(size_t seq, size_t n_heads, size_t hd) {
          seq * n_heads >= 950 && (seq + 15) / 16 * n_heads <= 512;
 }
 
+bool attention_prefill_spills(size_t seq) { return seq > static_cast<size_t>(kScoreLds); }
+
 // Sized by the kernel that takes the shape: a long prompt on the tiled kernel
 // needs its slots only (32 heads x 16384 positions 3.2 GB), not the one-launch
 // kernel's score rows (34 GB).

@@ -443,7 +443,7 @@ int prana_attention_prefill(const float* q, const float* k, const float* v, size
     Scratch& sc = scratch();
     std::lock_guard<std::mutex> lk(sc.mu);
     const size_t need = attention_prefill_scratch_floats(seq, n_heads, head_dim, prefill_tile_aligned(q, k));
-    int rc = sc.att.ensure(need * 4);
+    int rc = sc.att.ensure_prefill(need, seq);
     if (rc) return rc;
     hipStream_t s = pick_stream(stream);
     rc = launch_attention_prefill(q, k, v, seq, n_heads, n_kv_heads, head_dim, out,

@@ -166,7 +166,7 @@ int Graph::execute(hipStream_t s, int* kind, size_t* node) {
   int rc;
   if (q_elems && ((rc = qa.ensure(q_elems)) || (rc = sa.ensure(q_elems / 32 * 4)) || (rc = sums.ensure(q_elems / 32 * 4))))
     return rc;
-  if (att_floats && (rc = scratch.ensure(att_floats * 4))) return rc;
+  if (att_floats && (rc = scratch.ensure_prefill(att_floats, n_tokens))) return rc;
   for (size_t i = 0; i < nodes.size(); i++) {
     if (nodes[i].has_value) continue;
     if ((rc = eval(i, s, kind, node))) {

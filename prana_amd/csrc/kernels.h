@@ -249,6 +249,8 @@ int launch_attention_cache(const float* q, const uint16_t* kc, const uint16_t* v
 // Also the dim slices per head a launch uses.
 size_t attention_scratch_floats(size_t n_q, size_t n_heads, size_t ctx_cap);
 size_t attention_prefill_scratch_floats(size_t seq, size_t n_heads, size_t hd, bool aligned);
+// Whether a prefill needs its scratch on every kernel (more than 4096 positions).
+bool attention_prefill_spills(size_t seq);
 // Whether a one-row cache window of `rows` rows takes the split path.
 bool attention_split_window(size_t rows, size_t hd);
 int attention_dim_slices(size_t n_q, size_t n_heads, size_t hd, size_t elem, bool aligned);

@@ -252,10 +252,11 @@ int Model::ensure_ws(size_t n_tok, size_t ctx_cap, bool prefill_attn) {
     ws.gen++;
   }
   // (the workspace's q and k are allocations: aligned)
-  size_t need = (prefill_attn ? attention_prefill_scratch_floats(n_tok, c.n_heads, c.head_dim, true)
-                              : attention_scratch_floats(n_tok, c.n_heads, ctx_cap)) * 4;
+  const size_t need = std::max<size_t>(prefill_attn ? attention_prefill_scratch_floats(n_tok, c.n_heads, c.head_dim, true)
+                                                    : attention_scratch_floats(n_tok, c.n_heads, ctx_cap), 1);
   const void* before = ws.scratch.p;
-  if ((rc = ws.scratch.ensure(std::max<size_t>(need, 4)))) return rc;
+  rc = prefill_attn ? ws.scratch.ensure_prefill(need, n_tok) : ws.scratch.ensure(need * 4);
+  if (rc) return rc;
   if (ws.scratch.p != before) ws.gen++;
   return kOk;
 }

@@ -21,6 +21,7 @@ int fail(int code, const std::string& msg) {
 }
 
 int hip_fail(hipError_t e, const char* what) {
+  (void)hipGetLastError();  // reported here; the next launch check must not find it
   set_error(std::string("HIP error in ") + what + ": " + hipGetErrorString(e));
   return e == hipErrorOutOfMemory ? kErrNoMem : kErrHip;
 }
@@ -74,6 +75,11 @@ int DevBuf::alloc(size_t n) {
 }
 
 int DevBuf::ensure(size_t n) { return n <= bytes ? kOk : alloc(n); }
+
+int DevBuf::ensure_prefill(size_t floats, size_t seq) {
+  const int rc = ensure(floats * 4);
+  return rc == kErrNoMem && !attention_prefill_spills(seq) ? kOk : rc;
+}
 
 float host_f16_to_f32(uint16_t h) {
   uint32_t sign = (h >> 15) & 1u, exp = (h >> 10) & 0x1fu, frac = h & 0x3ffu;

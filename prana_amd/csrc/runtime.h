@@ -49,6 +49,10 @@ struct DevBuf {
   ~DevBuf();
   int alloc(size_t n);  // frees the previous allocation
   int ensure(size_t n);  // grow-only
+  // A prefill's score rows (attention_prefill_scratch_floats): where the
+  // memory left does not hold them and the window does without, the buffer
+  // stays empty and the one-launch kernel runs.
+  int ensure_prefill(size_t floats, size_t seq);
   template <class T>
   T* as() const {
     return static_cast<T*>(p);

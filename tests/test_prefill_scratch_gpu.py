@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import prana_amd as P
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -25,3 +26,28 @@ def test_prefill_scratch_is_the_kernels_own(seq, nh, nkv, hd, slot_rows):
     taken = free - torch.cuda.mem_get_info()[0]
     want = 4 * (slot_rows * -(-seq // STRIDE) * STRIDE + seq * nh * hd)
     assert want // 2 < taken < want + (32 << 20), (taken, want)  # (allocations come in pages of a few MiB)
+
+
+def test_prefill_without_room_for_scratch():
+    # 403 MB of score rows with about 250 MB left: the window runs without
+    seq, nh, nkv, hd = 2048, 32, 32, 4
+    r = np.random.default_rng(3)
+    host = [r.standard_normal((seq, n * hd)).astype(np.float32) for n in (nh, nkv, nkv)]
+    g = P.Graph()
+    nodes = [g.input(seq) for _ in range(3)]
+    out = g.attention(*nodes, nh, nkv, hd)
+    for node, a in zip(nodes, host):
+        g.set_input(node, a)
+    torch.cuda.empty_cache()
+    try:
+        held = torch.empty(torch.cuda.mem_get_info()[0] - (250 << 20), dtype=torch.uint8, device="cuda")
+    except torch.OutOfMemoryError:
+        pytest.skip("the card's free memory is not one piece")
+    try:
+        g.execute()
+    finally:
+        del held
+        torch.cuda.empty_cache()
+    got = np.asarray(g.output_f32(out), np.float32)
+    want = O.attention(*(a.ravel() for a in host), seq, nh, nkv, hd)
+    assert np.array_equal(got.ravel().view(np.uint32), np.asarray(want, np.float32).ravel().view(np.uint32))
