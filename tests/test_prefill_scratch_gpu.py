@@ -29,7 +29,7 @@ def test_prefill_scratch_is_the_kernels_own(seq, nh, nkv, hd, slot_rows):
 
 
 def test_prefill_without_room_for_scratch():
-    # 403 MB of score rows with about 250 MB left: the window runs without
+    # 403 MB of score rows with about 200 MB left: the window runs without
     seq, nh, nkv, hd = 2048, 32, 32, 4
     r = np.random.default_rng(3)
     host = [r.standard_normal((seq, n * hd)).astype(np.float32) for n in (nh, nkv, nkv)]
@@ -39,15 +39,23 @@ def test_prefill_without_room_for_scratch():
     for node, a in zip(nodes, host):
         g.set_input(node, a)
     torch.cuda.empty_cache()
+    piece = 64 << 20
+    held = []
     try:
-        held = torch.empty(torch.cuda.mem_get_info()[0] - (250 << 20), dtype=torch.uint8, device="cuda")
-    except torch.OutOfMemoryError:
-        pytest.skip("the card's free memory is not one piece")
+        # (the free memory that is reported and what can be allocated differ by a few pieces)
+        held.append(P.DeviceArray((torch.cuda.mem_get_info()[0] - 2 * piece,), np.uint8))
+        for _ in range(64):
+            held.append(P.DeviceArray((piece,), np.uint8))
+    except P.PranaError:
+        pass
+    if not 4 < len(held) < 65:
+        pytest.skip("free memory of this card cannot be narrowed down")
+    del held[-3:]
     try:
         g.execute()
     finally:
-        del held
-        torch.cuda.empty_cache()
+        print("pieces", len(held))
+        held.clear()
     got = np.asarray(g.output_f32(out), np.float32)
     want = O.attention(*(a.ravel() for a in host), seq, nh, nkv, hd)
     assert np.array_equal(got.ravel().view(np.uint32), np.asarray(want, np.float32).ravel().view(np.uint32))
