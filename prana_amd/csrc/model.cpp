@@ -234,6 +234,7 @@ int Model::ensure_ws(size_t n_tok, size_t ctx_cap, bool prefill_attn) {
   if (n_tok > ws.cap_tok) {
     size_t n = n_tok;
     ws.gen++;
+    ws.cap_tok = 0;  // until every buffer stands: a failed allocation leaves some of them empty
     if ((rc = ws.x.alloc(n * c.dim * 4)) || (rc = ws.xb.alloc(n * c.dim * 4)) || (rc = ws.q.alloc(n * q_dim * 4)) ||
         (rc = ws.k.alloc(n * kv_dim * 4)) || (rc = ws.v.alloc(n * kv_dim * 4)) ||
         (rc = ws.attn.alloc(n * q_dim * 4)) || (rc = ws.gate.alloc(n * c.hidden_dim * 4)) ||

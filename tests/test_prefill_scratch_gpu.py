@@ -8,6 +8,7 @@ import torch
 
 import prana_amd as P
 from oracle import oracle as O
+from prana_amd import models as M
 
 pytestmark = pytest.mark.gpu
 
@@ -28,16 +29,8 @@ def test_prefill_scratch_is_the_kernels_own(seq, nh, nkv, hd, slot_rows):
     assert want // 2 < taken < want + (32 << 20), (taken, want)  # (allocations come in pages of a few MiB)
 
 
-def test_prefill_without_room_for_scratch():
-    # 403 MB of score rows with about 200 MB left: the window runs without
-    seq, nh, nkv, hd = 2048, 32, 32, 4
-    r = np.random.default_rng(3)
-    host = [r.standard_normal((seq, n * hd)).astype(np.float32) for n in (nh, nkv, nkv)]
-    g = P.Graph()
-    nodes = [g.input(seq) for _ in range(3)]
-    out = g.attention(*nodes, nh, nkv, hd)
-    for node, a in zip(nodes, host):
-        g.set_input(node, a)
+def leave_little_memory():
+    """Buffers that leave about 200 MB of the card's memory."""
     torch.cuda.empty_cache()
     piece = 64 << 20
     held = []
@@ -50,12 +43,42 @@ def test_prefill_without_room_for_scratch():
         pass
     if not 4 < len(held) < 65:
         pytest.skip("free memory of this card cannot be narrowed down")
-    del held[-3:]
+    return held[:-3]
+
+
+def test_prefill_without_room_for_scratch():
+    # 403 MB of score rows with about 200 MB left: the window runs without
+    seq, nh, nkv, hd = 2048, 32, 32, 4
+    r = np.random.default_rng(3)
+    host = [r.standard_normal((seq, n * hd)).astype(np.float32) for n in (nh, nkv, nkv)]
+    g = P.Graph()
+    nodes = [g.input(seq) for _ in range(3)]
+    out = g.attention(*nodes, nh, nkv, hd)
+    for node, a in zip(nodes, host):
+        g.set_input(node, a)
+    held = leave_little_memory()
     try:
         g.execute()
     finally:
-        print("pieces", len(held))
         held.clear()
     got = np.asarray(g.output_f32(out), np.float32)
     want = O.attention(*(a.ravel() for a in host), seq, nh, nkv, hd)
     assert np.array_equal(got.ravel().view(np.uint32), np.asarray(want, np.float32).ravel().view(np.uint32))
+
+
+def test_model_runs_on_after_a_batch_that_does_not_fit():
+    # a prompt whose logits (1.2 GB) do not fit is refused, and the next call
+    # finds its buffers again
+    cfg = M.config(64, 96, 1, 2, 2, 100000, 3000, head_dim=32)
+    t = M.synth_tensors(cfg, lambda name, cols: P.Q8_0, 9)
+    g, o = P.Model(cfg, t), O.Model(cfg, t)
+    gc, oc = g.cache(3000), o.cache(3000)
+    assert np.array_equal(gc.forward(5, 0), oc.forward(5, 0))
+    held = leave_little_memory()
+    try:
+        with pytest.raises(P.PranaError) as e:
+            gc.prefill(np.zeros(3000, np.uint32))
+        assert e.value.code == -3  # PRANA_ERR_NOMEM
+        assert np.array_equal(gc.forward(7, 1), oc.forward(7, 1))
+    finally:
+        held.clear()
